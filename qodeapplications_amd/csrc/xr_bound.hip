@@ -439,7 +439,7 @@ extern "C" int xr_cholesky_test(xr_ctx* c, int nb, const int64_t* n, double* con
             }
         }
         if (!narrow.empty()) {
-            const int rc = launch_grouped<128, 64>(c, narrow, 0, 1, Ms.data(), Ns.data(), Ks.data(), 1.0, As.data(),
+            const int rc = launch_grouped_any<128, 64>(c, narrow, 0, 1, Ms.data(), Ns.data(), Ks.data(), 1.0, As.data(),
                                                    lda.data(), Bs.data(), ldb.data(), Cs.data(), ldc.data(), 0.0, 0,
                                                    XR_K_OTHER);
             if (rc) return rc;
@@ -462,7 +462,7 @@ extern "C" int xr_cholesky_test(xr_ctx* c, int nb, const int64_t* n, double* con
             r++;
         }
         if (!wide.empty()) {
-            const int rc = launch_grouped<128, 128>(c, wide, 0, 1, Ms.data(), Ms.data(), Ks.data(), -1.0, Ws.data(),
+            const int rc = launch_grouped_any<128, 128>(c, wide, 0, 1, Ms.data(), Ms.data(), Ks.data(), -1.0, Ws.data(),
                                                     ldc.data(), Ws.data(), ldc.data(), Cu.data(), ldu.data(), 1.0, 1,
                                                     XR_K_OTHER);
             if (rc) return rc;

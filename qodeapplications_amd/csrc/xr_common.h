@@ -121,6 +121,10 @@ struct xr_ctx {
     // side-adjoint index tables (one int32 code per source determinant and
     // tuple), keyed by the side string and the spaces it maps between
     std::map<std::array<int64_t, 12>, std::pair<int32_t*, int64_t>> sidetab;
+    // tile and K split chosen for recent product sizes (launch_chosen)
+    struct GemmChoice { std::array<int64_t, 5> key{-1, -1, -1, -1, -1}; int tile = 3; int64_t splits = 1, staging = 0; };
+    std::vector<GemmChoice> gemm_choice;
+    int64_t gemm_staging = 0;   // largest staging admitted since the last trim (gemm_admit)
     // GEMM autotune table: (ta, tb, M, N, K, batch) -> (tile, splits)
     std::map<std::array<int64_t, 6>, std::pair<int, int>> tune;
     // captured graphs holding the workspace addresses (xr_pin): while > 0 a
@@ -159,6 +163,7 @@ struct ProfScope {
 };
 int xr_hip_check(xr_ctx* c, hipError_t e, const char* what);
 void* xr_workspace(xr_ctx* c, int slot, size_t bytes);
+bool xr_workspace_fits(xr_ctx* c, int slot, size_t bytes);
 int xr_noalloc_init(xr_ctx* c);
 int xr_fill(xr_ctx* c, double* p, int64_t n, double v);
 

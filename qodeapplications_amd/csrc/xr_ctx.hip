@@ -29,6 +29,19 @@ int xr_hip_check(xr_ctx* c, hipError_t e, const char* what) {
 
 // Returns a device buffer of at least `bytes` for scratch slot `slot`,
 // growing it when needed (the old contents are not kept).
+// Whether xr_workspace would serve `bytes` from this slot as far as the
+// caps go (nothing is allocated).
+bool xr_workspace_fits(xr_ctx* c, int slot, size_t bytes) {
+    if (c->noalloc) return c->scratch && bytes <= c->scratch_bytes;
+    if ((int)c->ws.size() > slot && c->ws[slot] && c->ws_size[slot] >= bytes) return true;
+    if (c->pins > 0) return false;
+    if (!c->ws_limit) return true;
+    size_t total = bytes;
+    for (size_t i = 0; i < c->ws_size.size(); i++)
+        if ((int)i != slot) total += c->ws_size[i];
+    return total <= c->ws_limit;
+}
+
 void* xr_workspace(xr_ctx* c, int slot, size_t bytes) {
     if (c->noalloc) {           // a no-allocation call: the static scratch array or nothing
         if (c->scratch && bytes <= c->scratch_bytes) return c->scratch;
@@ -92,6 +105,7 @@ extern "C" int xr_trim(xr_ctx* c) {
         c->ws[i] = nullptr;
         c->ws_size[i] = 0;
     }
+    c->gemm_staging = 0;
     return XR_OK;
 }
 

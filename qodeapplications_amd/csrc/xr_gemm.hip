@@ -1,22 +1,20 @@
 // FP64 GEMM on the CDNA4 matrix cores (v_mfma_f64_16x16x4f64).
 //
-// C_b = alpha * op(A_b) op(B_b) + beta * C_b.  The tile kernel computes
-// alpha * op(A) op(B) only (alpha is applied while A is staged in LDS) and
-// stores the accumulators untouched: any arithmetic on them in the epilogue
-// makes the compiler copy all 128 accumulator registers out of the AGPRs,
-// which halves occupancy.  Split-K goes through a workspace and a
-// fixed-order reduction, and so does beta != 0 unless the accumulating
-// variant (k_dgemm_acc) costs nothing extra: small grids or short K.  256 threads = 4 waves per
-// workgroup in a 2 x 2 arrangement; each wave owns a (BM/2) x (BN/2) block of
-// 16 x 16 MFMA tiles.  K advances 16 at a time through one LDS stage while the
-// next stage is prefetched into registers.  Workgroups are remapped so each
-// XCD (own L2) receives a contiguous run of output tiles.
+// C_b = alpha * op(A_b) op(B_b) + beta * C_b.  Split-K goes through a
+// workspace and a fixed-order reduction; an unsplit product applies alpha and
+// beta where it stores C.  256 threads = 4 waves per workgroup, whose 16-row
+// (or 32-row) fragments of the output tile are dealt out to the waves in
+// turn.  K advances 16 at a time through two LDS stages, one barrier per step.
+// Workgroups are remapped so each XCD (own L2) receives a contiguous run of
+// output tiles.
 #include "xr_common.h"
 #include "xr_gemm.h"
 #include <vector>
 #include <algorithm>
+#include <type_traits>
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
+typedef double d2_t __attribute__((ext_vector_type(2)));
 
 #define GEMM_BK 16
 #define GEMM_THREADS 256
@@ -34,92 +32,197 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t total) {
     return base + j;
 }
 
-// Staged operand tiles are k-major with rows of BM (BN) + 16 doubles, so
-// rows k and k + 1 fall in opposite halves of the 64 LDS banks and the MFMA
-// fragment reads (16 lanes over the column, rows k and k + 1 per half-wave)
-// touch 32 distinct 8-byte bank pairs.  An operand that arrives K-fastest
-// from global memory (A not transposed, B transposed) is stored with 16
-// lanes over k: there the column's bits 1..3 are XORed with (k >> 1) & 7,
-// which spreads those stores over distinct bank pairs too; the reads apply
-// the same XOR (its ks part is a compile-time constant of the unrolled loop).
-__device__ __forceinline__ int lds_swz(int k, int col) {
-    return col ^ (((k >> 1) & 7) << 1);
-}
+// 16 bytes of zeros: where a load of a tile's padding (k past K) points.
+static __device__ __align__(16) double xr_zero_page[2] = {0.0, 0.0};
 
-// One BM x BN output tile at (m0, n0): C = alpha op(A) op(B) over [0, K),
-// or C = alpha op(A) op(B) + beta C with ACC (an epilogue that reads C costs
-// the accumulators' AGPR residency, so only the accumulating variant has it).
-template <int BM, int BN, bool TA, bool TB, bool ACC = false>
+// One operand of a tile: BX rows of op(A) (columns of op(B)) by 16 of k.
+// KC: K is contiguous in memory (A as stored, B transposed); otherwise the
+// BX index is.  LDS layout, in 16-byte chunks of two doubles:
+//   KC   row x holds its 8 chunks of k, chunk c at slot c ^ (x & 7);
+//   !KC  row k holds BX doubles.
+// Fragment reads are 16 bytes: with KC a lane takes two k of one row, else
+// two neighbouring rows x of one k.  A product over k may take its k in any
+// order that both operands share, so lane group fk supplies k = 8 s + 2 fk + h
+// to MFMA (s, h).  The slot XOR puts the 64 lanes of a KC read on distinct
+// banks (rows are 128 bytes apart, so without it 8 rows share one).
+//
+// DIRECT: the chunks go from memory straight into LDS
+// (global_load_lds_dwordx4: no staging registers, no LDS stores), which needs
+// 16-byte aligned rows: base, leading dimension and the extent along the
+// contiguous index even.  Otherwise 8-byte loads pass through registers.
+// Rows past the edge read the last row again (their results are not
+// stored); k past K reads the zero page.
+template <int BX, bool KC, bool DIRECT>
+struct TileOperand {
+    static constexpr int NI = BX / 32;                    // DIRECT: load instructions per wave and stage
+    static constexpr int NE = BX * GEMM_BK / GEMM_THREADS;   // registers: elements per thread and stage
+    const double* p[DIRECT ? NI : 1];
+    const double* base;
+    double r[DIRECT ? 1 : NE];
+    int64_t ld, x0, X;
+    int kofs[DIRECT ? NI : 1];
+
+    __device__ __forceinline__ void init(const double* src, int64_t ld_, int64_t x0_, int64_t X_, int lane, int wave) {
+        base = src;
+        ld = ld_;
+        x0 = x0_;
+        X = X_;
+        if constexpr (DIRECT) {
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                if (KC) {
+                    int64_t x = x0 + wave * (BX / 4) + i * 8 + (lane >> 3);
+                    if (x > X - 1) x = X - 1;
+                    kofs[i] = 2 * ((lane & 7) ^ (lane >> 3));
+                    p[i] = src + x * ld + kofs[i];
+                } else {
+                    int64_t x = x0 + 2 * (lane % (BX / 2));
+                    if (x > X - 2) x = X - 2;
+                    kofs[i] = (wave * NI + i) * (128 / BX) + lane / (BX / 2);
+                    p[i] = src + kofs[i] * ld + x;
+                }
+            }
+        }
+    }
+    // DIRECT: queues the loads of the next 16 k into `dst`; tail: only the
+    // first `krest` of them exist.  (The empty asm keeps the two branches
+    // apart: merged, every load of every stage pays the tail's selects.)
+    __device__ __forceinline__ void stage(double* dst, bool tail, int krest, int wave) {
+        auto go = [&](int i, const double* q) {
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)q,
+                                             (__attribute__((address_space(3))) void*)(dst + (wave * NI + i) * 128),
+                                             16, 0, 0);
+        };
+        if (tail) {
+            asm volatile("");
+#pragma unroll
+            for (int i = 0; i < NI; i++) go(i, kofs[i] < krest ? p[i] : xr_zero_page);
+            asm volatile("");
+        } else {
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                go(i, p[i]);
+                p[i] += KC ? GEMM_BK : GEMM_BK * ld;
+            }
+        }
+    }
+    // registers: loads of k in [k0, k0 + 16), then their LDS stores.  The
+    // first krest of them exist.
+    __device__ __forceinline__ void load(int64_t k0, int krest, int tid) {
+        if (KC) {
+            const int k = tid & 15, xlast = (int)(X - x0 < BX ? X - x0 : BX) - 1;
+            int x = tid >> 4;
+            int64_t off = (x0 + (x < xlast ? x : xlast)) * ld + k0 + k;
+#pragma unroll
+            for (int i = 0; i < NE; i++) {
+                const double* q = base + off;
+                if (k >= krest) q = xr_zero_page;
+                r[i] = *q;
+                const int up = xlast - x < 16 ? xlast - x : 16;   // rows left below the clamp
+                off += (up > 0 ? up : 0) * ld;
+                x += 16;
+                asm("" : "+v"(off));
+            }
+        } else {
+            int64_t x = x0 + tid % BX;
+            if (x > X - 1) x = X - 1;
+            int k = tid / BX;
+            int64_t off = (k0 + k) * ld + x;
+#pragma unroll
+            for (int i = 0; i < NE; i++) {
+                const double* q = base + off;
+                if (k >= krest) q = xr_zero_page;
+                r[i] = *q;
+                off += (GEMM_THREADS / BX) * ld;
+                k += GEMM_THREADS / BX;
+                asm("" : "+v"(off));           // one running offset, not one kept register pair per row
+            }
+        }
+    }
+    __device__ __forceinline__ void store(double* dst, int tid) {
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            if (KC) {
+                const int k = tid & 15, x = (tid >> 4) + 16 * i;
+                dst[x * GEMM_BK + 2 * ((k >> 1) ^ (x & 7)) + (k & 1)] = r[i];
+            } else {
+                dst[(tid / BX + i * (GEMM_THREADS / BX)) * BX + tid % BX] = r[i];
+            }
+        }
+    }
+};
+
+// Fragments of one operand for a wave: F MFMA fragments of 16 rows.  KC:
+// fragment f covers rows (2 f + w) 16 + [0, 16).  !KC: fragments 2 g and
+// 2 g + 1 cover the even and odd rows of (2 g + w) 32 + [0, 32).
+template <int F, int BX, bool KC>
+struct TileFrags {
+    d2_t v[GEMM_BK / 8][F];       // KC: [s][f] = k pair;  !KC: [s][2 g + h] = row pair at k parity h
+    __device__ __forceinline__ void read(const double* src, int w, int fr, int fk, int s) {
+#pragma unroll
+        for (int f = 0; f < F; f++) {
+            if (KC) {
+                const int x = (2 * f + w) * 16 + fr;
+                v[s][f] = *(const d2_t*)(src + x * GEMM_BK + 2 * ((4 * s + fk) ^ (fr & 7)));
+            } else {
+                const int k = 8 * s + 2 * fk + (f & 1);
+                v[s][f] = *(const d2_t*)(src + k * BX + (f - (f & 1) + w) * 32 + 2 * fr);
+            }
+        }
+    }
+    __device__ __forceinline__ double get(int s, int h, int f) const {
+        return KC ? v[s][f][h] : v[s][f - (f & 1) + h][f & 1];
+    }
+    // fragments that touch rows below `rem`
+    static __device__ __forceinline__ int valid(int64_t rem, int w) {
+        int n = 0;
+#pragma unroll
+        for (int f = 0; f < F; f++) n += (KC ? (2 * f + w) * 16 : (f - (f & 1) + w) * 32) < rem ? 1 : 0;
+        return n;
+    }
+    // row of element i (0..15) of fragment f
+    static __device__ __forceinline__ int row(int f, int w, int i) {
+        return KC ? (2 * f + w) * 16 + i : (f - (f & 1) + w) * 32 + 2 * i + (f & 1);
+    }
+};
+
+// One BM x BN output tile at (m0, n0): C = alpha op(A) op(B) + beta C over [0, K).
+//
+// Bound by the matrix cores: a 16-deep step of a 128 x 128 tile is 64 MFMAs
+// of 64 cycles per wave against 8 load instructions and 16 LDS reads.  The
+// order inside a step keeps everything else off that path: the barrier
+// that ends the previous step, all fragment reads of this stage, then the
+// loads of the next stage (after the reads: the compiler makes a read wait
+// for every load into LDS queued before it), then the MFMAs.  The accumulators live
+// in ordinary registers (220 of 256 at two waves per SIMD), so alpha and beta
+// cost nothing at the store.  Measured on 8192^3: 73.4 TFLOP/s (0.93 of
+// the FP64 matrix peak), against 59.7 with guarded 8-byte loads through
+// registers and two barriers per step.
+// Fragments wholly past M or N are skipped, and neighbouring fragments
+// belong to different waves, so an edge tile costs about its valid 16 or 32 row
+// groups on every SIMD rather than the whole tile.
+template <int BM, int BN, bool TA, bool TB, bool DIRECT>
 __device__ __forceinline__ void dgemm_tile(int64_t M, int64_t N, int64_t K, double alpha,
                                            const double* __restrict__ A, int64_t lda,
                                            const double* __restrict__ B, int64_t ldb,
                                            double* __restrict__ C, int64_t ldc, int64_t m0, int64_t n0,
                                            double beta = 0.0) {
-    constexpr int WM = BM / 2, WN = BN / 2;    // wave tile
-    constexpr int FM = WM / 16, FN = WN / 16;  // MFMA tiles per wave
-    constexpr int A_PER = BM * GEMM_BK / GEMM_THREADS;
-    constexpr int B_PER = BN * GEMM_BK / GEMM_THREADS;
-    constexpr int SA = BM + 16, SB = BN + 16;  // LDS row strides (doubles)
-    constexpr bool XA = !TA, XB = TB;          // operands stored with the column XOR
-    __shared__ double As[GEMM_BK * SA];
-    __shared__ double Bs[GEMM_BK * SB];
+    constexpr int FM = BM / 32, FN = BN / 32;  // MFMA fragments per wave and side
+    __shared__ __align__(1024) double As[2][BM * GEMM_BK];
+    __shared__ __align__(1024) double Bs[2][BN * GEMM_BK];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-
-    double ra[A_PER], rb[B_PER];
-
-    auto load_a = [&](int64_t k0) {
-#pragma unroll
-        for (int i = 0; i < A_PER; i++) {
-            int mm, kk;
-            if (TA) {  // A[k][m]
-                mm = tid % BM;
-                kk = tid / BM + i * (GEMM_THREADS / BM);
-            } else {   // A[m][k]
-                kk = tid % GEMM_BK;
-                mm = tid / GEMM_BK + i * (GEMM_THREADS / GEMM_BK);
-            }
-            int64_t gm = m0 + mm, gk = k0 + kk;
-            double v = 0.0;
-            if (gm < M && gk < K) v = TA ? A[gk * lda + gm] : A[gm * lda + gk];
-            ra[i] = v;
-        }
-    };
-    auto load_b = [&](int64_t k0) {
-#pragma unroll
-        for (int i = 0; i < B_PER; i++) {
-            int nn, kk;
-            if (!TB) {  // B[k][n]
-                nn = tid % BN;
-                kk = tid / BN + i * (GEMM_THREADS / BN);
-            } else {    // B[n][k]
-                kk = tid % GEMM_BK;
-                nn = tid / GEMM_BK + i * (GEMM_THREADS / GEMM_BK);
-            }
-            int64_t gn = n0 + nn, gk = k0 + kk;
-            double v = 0.0;
-            if (gn < N && gk < K) v = TB ? B[gn * ldb + gk] : B[gk * ldb + gn];
-            rb[i] = v;
-        }
-    };
-    auto store_ab = [&]() {
-#pragma unroll
-        for (int i = 0; i < A_PER; i++) {
-            int mm, kk;
-            if (TA) { mm = tid % BM; kk = tid / BM + i * (GEMM_THREADS / BM); }
-            else { kk = tid % GEMM_BK; mm = tid / GEMM_BK + i * (GEMM_THREADS / GEMM_BK); }
-            As[kk * SA + (XA ? lds_swz(kk, mm) : mm)] = alpha * ra[i];
-        }
-#pragma unroll
-        for (int i = 0; i < B_PER; i++) {
-            int nn, kk;
-            if (!TB) { nn = tid % BN; kk = tid / BN + i * (GEMM_THREADS / BN); }
-            else { kk = tid % GEMM_BK; nn = tid / GEMM_BK + i * (GEMM_THREADS / GEMM_BK); }
-            Bs[kk * SB + (XB ? lds_swz(kk, nn) : nn)] = rb[i];
-        }
-    };
+    const int fr = lane & 15;   // row / column inside a fragment
+    const int fk = lane >> 4;   // k group of a fragment
+    typedef TileFrags<FM, BM, !TA> FragA;
+    typedef TileFrags<FN, BN, TB> FragB;
+    TileOperand<BM, !TA, DIRECT> oa;
+    TileOperand<BN, TB, DIRECT> ob;
+    oa.init(A, lda, m0, M, lane, wave);
+    ob.init(B, ldb, n0, N, lane, wave);
+    const int fmv = FragA::valid(M - m0, wm), fnv = FragB::valid(N - n0, wn);
 
     d4_t acc[FM][FN];
 #pragma unroll
@@ -127,90 +230,157 @@ __device__ __forceinline__ void dgemm_tile(int64_t M, int64_t N, int64_t K, doub
 #pragma unroll
         for (int j = 0; j < FN; j++) acc[i][j] = d4_t{0.0, 0.0, 0.0, 0.0};
 
-    const int64_t nk = (K + GEMM_BK - 1) / GEMM_BK;
-    if (nk > 0) {
-        load_a(0);
-        load_b(0);
-        store_ab();
-        __syncthreads();
-    }
-    const int fr = lane & 15;   // row / column inside a 16-wide fragment
-    const int fk = lane >> 4;   // k inside a 4-deep step
-    // fragment read offsets per 4-deep step ks: row ks*4 + fk, column
-    // (w*W + i*16 + fr) with the XOR of row (ks*4 + fk), whose ks part is
-    // 4 ks on the column's bits 2..3
-    int aoff[GEMM_BK / 4], boff[GEMM_BK / 4];
+    FragA fa;
+    FragB fb;
+    // FULL: every fragment of the wave is inside; k outermost, so the first
+    // MFMAs wait for the first fragments only.  Else skip the outside ones.
+    auto mults = [&](auto FULL, int s0, int s1) {
+        if constexpr (FULL.value) {
 #pragma unroll
-    for (int ks = 0; ks < GEMM_BK / 4; ks++) {
-        const int x = ((2 * ks + (fk >> 1)) & 7) << 1;
-        aoff[ks] = fk * SA + wm * WM + (XA ? (fr ^ x) : fr);
-        boff[ks] = fk * SB + wn * WN + (XB ? (fr ^ x) : fr);
-    }
-    for (int64_t kt = 0; kt < nk; kt++) {
-        if (kt + 1 < nk) {
-            load_a((kt + 1) * GEMM_BK);
-            load_b((kt + 1) * GEMM_BK);
-        }
+            for (int s = s0; s < s1; s++)
 #pragma unroll
-        for (int ks = 0; ks < GEMM_BK / 4; ks++) {
-            double af[FM], bf[FN];
+                for (int h = 0; h < 2; h++)
 #pragma unroll
-            for (int i = 0; i < FM; i++) af[i] = As[ks * 4 * SA + aoff[ks] + i * 16];
+                    for (int i = 0; i < FM; i++)
 #pragma unroll
-            for (int j = 0; j < FN; j++) bf[j] = Bs[ks * 4 * SB + boff[ks] + j * 16];
+                        for (int j = 0; j < FN; j++)
+                            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa.get(s, h, i), fb.get(s, h, j),
+                                                                             acc[i][j], 0, 0, 0);
+        } else {
 #pragma unroll
             for (int i = 0; i < FM; i++)
 #pragma unroll
-                for (int j = 0; j < FN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < FN; j += 2)
+                    if (i < fmv && j < fnv) {
+#pragma unroll
+                        for (int s = s0; s < s1; s++)
+#pragma unroll
+                            for (int h = 0; h < 2; h++)
+#pragma unroll
+                                for (int e = 0; e < 2; e++)
+                                    acc[i][j + e] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                                        fa.get(s, h, i), fb.get(s, h, j + e), acc[i][j + e], 0, 0, 0);
+                    }
         }
-        __syncthreads();
-        if (kt + 1 < nk) {
-            store_ab();
-            __syncthreads();
+    };
+    const int steps = (int)((K + GEMM_BK - 1) / GEMM_BK);
+    const int klast = (int)(K - (int64_t)(steps - 1) * GEMM_BK);      // k of the last step, 1..16
+    auto queue = [&](int buf, int t) {         // the loads of step t into stage buf
+        const bool tail = t == steps - 1 && klast < GEMM_BK;
+        if constexpr (DIRECT) {
+            oa.stage(As[buf], tail, klast, wave);
+            ob.stage(Bs[buf], tail, klast, wave);
+        } else {
+            oa.load((int64_t)t * GEMM_BK, tail ? klast : GEMM_BK, tid);
+            ob.load((int64_t)t * GEMM_BK, tail ? klast : GEMM_BK, tid);
         }
+    };
+    auto land = [&](int buf) {                 // registers only: the queued values into LDS
+        if constexpr (!DIRECT) {
+            oa.store(As[buf], tid);
+            ob.store(Bs[buf], tid);
+        }
+    };
+    auto step = [&](auto FULL, int cur, int tnext) {
+        __syncthreads();                       // this stage is in LDS, the other one is free
+        if constexpr (DIRECT) {
+#pragma unroll
+            for (int s = 0; s < GEMM_BK / 8; s++) {
+                fa.read(As[cur], wm, fr, fk, s);
+                fb.read(Bs[cur], wn, fr, fk, s);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (tnext < steps) queue(cur ^ 1, tnext);
+            __builtin_amdgcn_sched_barrier(0);
+            mults(FULL, 0, GEMM_BK / 8);
+        } else {
+            // the staging registers leave room for the fragments of 8 k only
+            if (tnext < steps) queue(cur ^ 1, tnext);
+#pragma unroll
+            for (int s = 0; s < GEMM_BK / 8; s++) {
+                __builtin_amdgcn_sched_barrier(0);
+                fa.read(As[cur], wm, fr, fk, s);
+                fb.read(Bs[cur], wn, fr, fk, s);
+                mults(FULL, s, s + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (tnext < steps) land(cur ^ 1);
+        }
+    };
+    if (steps > 0) {
+        queue(0, 0);
+        land(0);
     }
+    // the same barriers in both loops: waves of one workgroup may take either
+    auto loop = [&](auto FULL) {
+        for (int t = 0; t < steps; t += 2) {
+            step(FULL, 0, t + 1);
+            if (t + 1 < steps) step(FULL, 1, t + 2);
+        }
+    };
+    if (fmv == FM && fnv == FN) loop(std::integral_constant<bool, true>());
+    else loop(std::integral_constant<bool, false>());
 
-    // D[row][col] of a 16x16 tile (v_mfma_f64_16x16x4f64, checked on gfx950):
-    // col = lane % 16, row = lane / 16 + 4 * r for accumulator element r.
-    // With ACC the C values of one row of MFMA tiles are all loaded before
-    // any is stored: loads and stores through the one C pointer would
-    // otherwise stay in program order, one memory round trip per element.
+    // D[row][col] of a 16x16 fragment (v_mfma_f64_16x16x4f64, checked on
+    // gfx950): col = lane % 16, row = lane / 16 + 4 * r for element r.
+    // All C values of a fragment row are loaded before any is stored: loads
+    // and stores through the one C pointer would otherwise stay in program order.
+    const bool pair = !TB && (ldc & 1) == 0 && ((uintptr_t)C & 15) == 0;   // fragments j, j + 1 adjacent in C
 #pragma unroll
     for (int i = 0; i < FM; i++) {
-        double cv[FN][4];
-        if (ACC) {
+        if (i >= fmv) continue;
+        d2_t cv[FN / 2][4];
+        if (beta != 0.0) {
 #pragma unroll
-            for (int j = 0; j < FN; j++)
+            for (int j = 0; j < FN; j += 2)
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const int64_t gm = m0 + wm * WM + i * 16 + fk + 4 * r;
-                    const int64_t gn = n0 + wn * WN + j * 16 + fr;
-                    cv[j][r] = (gm < M && gn < N) ? C[gm * ldc + gn] : 0.0;
+                    const int64_t gm = m0 + FragA::row(i, wm, fk + 4 * r);
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        const int64_t gn = n0 + FragB::row(j + e, wn, fr);
+                        cv[j / 2][r][e] = (gm < M && gn < N) ? C[gm * ldc + gn] : 0.0;
+                    }
                 }
         }
 #pragma unroll
-        for (int j = 0; j < FN; j++)
+        for (int j = 0; j < FN; j += 2)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int64_t gm = m0 + wm * WM + i * 16 + fk + 4 * r;
-                const int64_t gn = n0 + wn * WN + j * 16 + fr;
-                if (gm < M && gn < N) {
-                    if (ACC) C[gm * ldc + gn] = acc[i][j][r] + beta * cv[j][r];
-                    else C[gm * ldc + gn] = acc[i][j][r];
+                const int64_t gm = m0 + FragA::row(i, wm, fk + 4 * r);
+                const int64_t gn = n0 + FragB::row(j, wn, fr), gn1 = n0 + FragB::row(j + 1, wn, fr);
+                d2_t v = {alpha * acc[i][j][r], alpha * acc[i][j + 1][r]};
+                if (beta != 0.0) v += beta * cv[j / 2][r];
+                if (gm < M) {
+                    if (pair && gn1 < N) {
+                        *(d2_t*)(C + gm * ldc + gn) = v;
+                    } else {
+                        if (gn < N) C[gm * ldc + gn] = v[0];
+                        if (gn1 < N) C[gm * ldc + gn1] = v[1];
+                    }
                 }
             }
     }
 }
 
+// Whether both operands' tiles can be loaded in 16-byte chunks (DIRECT):
+// base, leading dimension, batch stride and the extent along the contiguous
+// index even.
+static inline bool gemm_direct(int ta, int tb, int64_t M, int64_t N, int64_t K, const double* A, int64_t lda,
+                               int64_t sA, const double* B, int64_t ldb, int64_t sB) {
+    const int64_t ea = ta ? M : K, eb = tb ? K : N;
+    return ((((uintptr_t)A | (uintptr_t)B) & 15) | ((lda | ldb | sA | sB | ea | eb) & 1)) == 0;
+}
 
-template <int BM, int BN, bool TA, bool TB>
-__global__ __launch_bounds__(GEMM_THREADS) void k_dgemm(
+// Waves per SIMD the register budget of a tile allows (LDS allows as many).
+#define GEMM_WAVES(BM, BN) ((BM) * (BN) >= 128 * 128 ? 2 : ((BM) * (BN) >= 128 * 64 ? 3 : 4))
+
+template <int BM, int BN, bool TA, bool TB, bool DIRECT>
+__global__ __launch_bounds__(GEMM_THREADS, GEMM_WAVES(BM, BN)) void k_dgemm(
     int64_t M, int64_t N, int64_t K, double alpha, const double* __restrict__ A, int64_t lda,
     int64_t sA, const double* __restrict__ B, int64_t ldb, int64_t sB, double beta,
     double* __restrict__ C, int64_t ldc, int64_t sC, int64_t tiles_m, int64_t tiles_n,
-    int64_t kchunk, int64_t sSplit, int upper = 0) {
-    (void)beta;
+    int64_t kchunk, int64_t sSplit, int upper) {
     const int64_t batch = blockIdx.z;
     A += batch * sA;
     B += batch * sB;
@@ -232,29 +402,128 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_dgemm(
     if (upper && tm > tn) return;              // symmetric product: the upper tiles only
     const int64_t m0 = tm * BM, n0 = tn * BN;
 
-    dgemm_tile<BM, BN, TA, TB>(M, N, K, alpha, A, lda, B, ldb, C, ldc, m0, n0);
+    dgemm_tile<BM, BN, TA, TB, DIRECT>(M, N, K, alpha, A, lda, B, ldb, C, ldc, m0, n0, beta);
 }
 
-// C_b = alpha op(A_b) op(B_b) + beta C_b without a K split, accumulating in
-// the epilogue (saves the workspace pass of the staged path for beta != 0).
-template <int BM, int BN, bool TA, bool TB>
-__global__ __launch_bounds__(GEMM_THREADS) void k_dgemm_acc(
-    int64_t M, int64_t N, int64_t K, double alpha, const double* __restrict__ A, int64_t lda,
-    int64_t sA, const double* __restrict__ B, int64_t ldb, int64_t sB, double beta,
-    double* __restrict__ C, int64_t ldc, int64_t sC, int64_t tiles_m, int64_t tiles_n) {
+// Small products: 32 x 32 output tiles, the four waves of a workgroup taking
+// every fourth 8-deep chunk of K and adding their tiles through LDS in wave order.
+// What bounds these is latency, not rate: a 64 x 64 tile that stages each
+// 16 of K behind a barrier takes 0.7 us a step with one workgroup per CU
+// whatever the tile holds.  Here a wave loads its fragments straight from
+// memory (L2) into registers, four chunks ahead of their use, waits for
+// nobody until the end, and does a quarter of K.
+template <bool TA, bool TB>
+__global__ __launch_bounds__(GEMM_THREADS) void k_dgemm_small(
+    int64_t M, int64_t N, int64_t K, double alpha, const double* __restrict__ A, int64_t lda, int64_t sA,
+    const double* __restrict__ B, int64_t ldb, int64_t sB, double beta, double* __restrict__ C, int64_t ldc,
+    int64_t sC, int tiles_n, int64_t kchunk, int64_t sSplit, int upper) {
+    const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
+    if (upper && tm > tn) return;
     const int64_t batch = blockIdx.z;
     A += batch * sA;
     B += batch * sB;
-    C += batch * sC;
-    const int64_t tile = xcd_remap(blockIdx.x, (int64_t)gridDim.x);
-    const int64_t GROUP = 8;
-    const int64_t per_group = GROUP * tiles_n;
-    const int64_t g = tile / per_group;
-    const int64_t first_m = g * GROUP;
-    const int64_t gsize = (tiles_m - first_m < GROUP) ? (tiles_m - first_m) : GROUP;
-    const int64_t tm = first_m + (tile % per_group) % gsize;
-    const int64_t tn = (tile % per_group) / gsize;
-    dgemm_tile<BM, BN, TA, TB, true>(M, N, K, alpha, A, lda, B, ldb, C, ldc, tm * BM, tn * BN, beta);
+    C += batch * sC + (int64_t)blockIdx.y * sSplit;
+    const int64_t kbeg = (int64_t)blockIdx.y * kchunk;
+    K = (K - kbeg < kchunk) ? (K - kbeg) : kchunk;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, fk = lane >> 4;
+    const int64_t m0 = (int64_t)tm * 32, n0 = (int64_t)tn * 32;
+    // element (row, k) of op(A) at pa[f] + k * ka; rows past the edge repeat the last one
+    const int64_t ka = TA ? lda : 1, kb = TB ? 1 : ldb;
+    const double* pa[2];
+    const double* pb[2];
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+        int64_t m = m0 + 16 * f + fr, n = n0 + 16 * f + fr;
+        if (m > M - 1) m = M - 1;
+        if (n > N - 1) n = N - 1;
+        pa[f] = A + (TA ? m : m * lda) + (kbeg + 8 * wave + 2 * fk) * ka;
+        pb[f] = B + (TB ? n * ldb : n) + (kbeg + 8 * wave + 2 * fk) * kb;
+    }
+    d4_t acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = d4_t{0.0, 0.0, 0.0, 0.0};
+    constexpr int U = 4;                       // chunks in flight
+    double a[U][2][2], b[U][2][2];
+    auto load = [&](int u) {
+#pragma unroll
+        for (int f = 0; f < 2; f++) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                a[u][f][h] = pa[f][h * ka];
+                b[u][f][h] = pb[f][h * kb];
+            }
+            pa[f] += 32 * ka;
+            pb[f] += 32 * kb;
+        }
+    };
+    auto mult = [&](int u) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][i][h], b[u][j][h], acc[i][j], 0, 0, 0);
+    };
+    const int64_t whole = K / 8;               // whole chunks: this wave's are wave, wave + 4, ...
+    int64_t left = whole > wave ? (whole - wave + 3) / 4 : 0;
+    if (left >= U) {
+#pragma unroll
+        for (int u = 0; u < U; u++) load(u);
+        left -= U;
+        for (; left >= U; left -= U) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                mult(u);
+                load(u);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) mult(u);
+    }
+#pragma unroll
+    for (int u = 0; u < U - 1; u++)
+        if (u < left) load(u);
+#pragma unroll
+    for (int u = 0; u < U - 1; u++)
+        if (u < left) mult(u);
+    if ((K & 7) && (whole & 3) == wave) {      // the last chunk's K % 8
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const bool in = 8 * whole + 2 * fk + h < K;
+                const double* qa = in ? pa[f] + h * ka : xr_zero_page;
+                const double* qb = in ? pb[f] + h * kb : xr_zero_page;
+                a[0][f][h] = *qa;
+                b[0][f][h] = *qb;
+            }
+        mult(0);
+    }
+    __shared__ double red[4][16][64];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) red[wave][(i * 2 + j) * 4 + r][lane] = acc[i][j][r];
+    __syncthreads();
+    // wave w finishes fragment (i, j) = (w >> 1, w & 1)
+    const int64_t gn = n0 + (wave & 1) * 16 + fr;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int64_t gm = m0 + (wave >> 1) * 16 + fk + 4 * r;
+        const int e = wave * 4 + r;
+        double v = alpha * ((red[0][e][lane] + red[1][e][lane]) + (red[2][e][lane] + red[3][e][lane]));
+        if (gm < M && gn < N) {
+            if (beta != 0.0) v += beta * C[gm * ldc + gn];
+            C[gm * ldc + gn] = v;
+        }
+    }
 }
 
 // Grouped GEMM: up to XR_GROUP_PROBS independent products C_q = alpha
@@ -276,12 +545,12 @@ struct GemmProb {
 struct GemmGroup {
     int n;
     int lower;           // square products whose strictly upper tiles are skipped
-    double alpha, beta;  // beta: the accumulating variant only
+    double alpha, beta;
     GemmProb p[XR_GROUP_PROBS];
 };
 
-template <int BM, int BN, bool TA, bool TB, bool ACC = false>
-__global__ __launch_bounds__(GEMM_THREADS) void k_dgemm_grouped(GemmGroup g) {
+template <int BM, int BN, bool TA, bool TB, bool DIRECT>
+__global__ __launch_bounds__(GEMM_THREADS, GEMM_WAVES(BM, BN)) void k_dgemm_grouped(GemmGroup g) {
     const int x = (int)(blockIdx.x & 7);
     int64_t j = blockIdx.x >> 3, local = -1;
     int q = 0;
@@ -312,8 +581,8 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_dgemm_grouped(GemmGroup g) {
         tm = first_m + (local % per_group) % gsize;
         tn = (local % per_group) / gsize;
     }
-    dgemm_tile<BM, BN, TA, TB, ACC>(P.M, P.N, P.K, g.alpha, P.A, P.lda, P.B, P.ldb, P.C, P.ldc, tm * BM, tn * BN,
-                                    g.beta);
+    dgemm_tile<BM, BN, TA, TB, DIRECT>(P.M, P.N, P.K, g.alpha, P.A, P.lda, P.B, P.ldb, P.C, P.ldc, tm * BM, tn * BN,
+                                       g.beta);
 }
 
 // C = alpha * sum_s P[s * step] + beta * C, summed in split order.
@@ -781,119 +1050,219 @@ static int launch_nn_gram(xr_ctx* c, int64_t M, int64_t N, int64_t K, double alp
     return XR_OK;
 }
 
-// K split for `units` output tiles on `slots` resident workgroups:
-// returns the best score (ideal time / modelled time) and the split.  Rounds
-// of resident workgroups each take K/s + 32 (per-workgroup start-up and
-// store, in k units); the reduction reads and writes (s + 1) M N doubles
-// against the product's 2 M N K flops (~46 flops per byte at the kernel's
-// rate).  Each split keeps at least kmin of K: 256 in general, 64 for a
-// narrow output (one row or column of tiles), whose partials are few bytes
-// next to the operand it streams.
-static double split_choice(int64_t units, int64_t slots, int64_t K, int64_t* splits, int64_t kmin = 256) {
-    auto score = [&](int64_t s) {
-        const double rounds = std::ceil((double)(units * s) / (double)slots);
-        const double ideal = (double)units * (double)K / (double)slots;
-        const double t = rounds * ((double)K / (double)s + 32.0);
-        return ideal / t / (1.0 + (s > 1 ? (double)(s + 1) * 46.0 / (double)K : 0.0));
-    };
-    double best = score(1);
+// ---------------------------------------------------------------------------
+// Choice of tile shape and K split
+// ---------------------------------------------------------------------------
+// Tile 0: 128 x 128, 1: 128 x 64, 2: 64 x 128, 3: 64 x 64, 4: 32 x 32 (k_dgemm_small).
+struct GemmTile { int bm, bn, resident; double eff, alone; };
+// resident: workgroups a CU holds; eff: share of the FP64 matrix peak with
+// the CU full; alone: us one 16-deep step takes over its MFMAs when a
+// workgroup has the CU to itself (load latency and the barrier).  Measured
+// on products of 64 x 324 x 64 to 8192^3 (68.8, 68.3, 68.1 and 66.4 TFLOP/s for tiles 0 to 3 on
+// 8192 x 8192 x 4096; 142, 80, 79 and 47 us for 64, 128, 128 and 256 workgroups of 1024^3).
+static const GemmTile GEMM_TILES[5] = {
+    {128, 128, 2, 0.90, 0.50}, {128, 64, 3, 0.89, 0.40}, {64, 128, 3, 0.89, 0.40}, {64, 64, 5, 0.87, 0.26}, {32, 32, 4, 0.60, 0.10}};
+#define GEMM_STAGING_MAX ((int64_t)64 << 20)   // bytes of split-K partial tiles
+
+static int device_cus() {
+    static const int n = [] {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+            (void)hipGetLastError();
+            return 256;
+        }
+        return cus > 0 ? cus : 256;
+    }();
+    return n;
+}
+
+// Modelled time (us) of a product with the given tile and K split.  The
+// busiest CU takes n = ceil(workgroups / CUs) of them: either its matrix
+// cores are busy throughout (padding past the 16-row and 32-column fragments is
+// skipped), or it waits out the steps of one workgroup after another.  A
+// split adds the reduction's launch and its traffic.
+static double gemm_cost(const GemmTile& t, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t s, bool upper,
+                        int cus) {
+    const int64_t tm = ceil_div(M, t.bm), tn = ceil_div(N, t.bn);
+    const int64_t tiles = upper ? tm * (tm + 1) / 2 : tm * tn;
+    const int64_t units = tiles * batch * s;
+    const double n = std::ceil((double)units / cus);
+    const double fill = (double)(ceil_div(M, 16) * 16) * (double)(ceil_div(N, 32) * 32) /
+                        ((double)(tm * t.bm) * (double)(tn * t.bn));
+    const double steps = std::ceil((double)K / (double)s / GEMM_BK);
+    const double step = t.bm * t.bn * (2.0 * GEMM_BK) / 128.0 / 2400.0;    // us of MFMA per step at full rate
+    const double busy = n * steps * step * std::min(1.0, fill) / t.eff;
+    const double wait = std::ceil(n / t.resident) * steps * (step + t.alone);
+    double us = 3.0 + std::max(busy, wait);
+    if (s > 1) us += 4.0 + (double)(s + 1) * 8.0 * M * N * batch / 4.0e6;
+    return us;
+}
+
+// The tile and K split of least modelled time among tiles [first, last].
+// Each split keeps at least 64 of K, and the partial tiles stay within the
+// staging array of the no-allocation entry point, so both entry points choose alike.
+static void gemm_choose(int64_t M, int64_t N, int64_t K, int64_t batch, bool direct, bool upper, int* tile,
+                        int64_t* splits) {
+    static const int S[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512};
+    const int cus = device_cus();
+    double best = 1e300;
+    *tile = 3;
     *splits = 1;
-    if (K < 512 || units >= 4 * slots) return best;
-    // up to two rounds of resident workgroups (at most 512 splits): a few
-    // output tiles over a long K are bound by how many CUs stream operands
-    const int64_t smax = std::min<int64_t>(std::min<int64_t>(512, std::max<int64_t>(64, 2 * slots / units)), K / kmin);
-    for (int64_t s = 2; s <= smax; s++) {
-        const double e = score(s);
-        if (e > best) { best = e; *splits = s; }
-    }
-    return best;
-}
-
-template <int BM, int BN>
-static int64_t tile_slots() {
-    static const int64_t r = resident_blocks(reinterpret_cast<const void*>(&k_dgemm<BM, BN, false, false>));
-    return r;
-}
-
-template <int BM, int BN>
-static int launch_tiles(xr_ctx* c, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                        const double* A, int64_t lda, int64_t sA, const double* B, int64_t ldb,
-                        int64_t sB, double beta, double* C, int64_t ldc, int64_t sC,
-                        int64_t batch, int splits_req = 0, bool upper = false) {
-    int64_t tm = ceil_div(M, BM), tn = ceil_div(N, BN);
-    int64_t tiles = tm * tn;
-    if (tiles > 0x7fffffff || batch > 65535)
-        return xr_fail(c, XR_EUNSUPPORTED, "GEMM grid too large");
-    // split K when the output tiles leave the last round of resident
-    // workgroups partly empty; the partial products go to scratch and are
-    // summed in a fixed order (deterministic)
-    int64_t splits = 1, kchunk = K;
-    if (splits_req > 0) {                    // from the autotune table
-        kchunk = ceil_div(ceil_div(K, splits_req), GEMM_BK) * GEMM_BK;
-        if (kchunk < GEMM_BK) kchunk = GEMM_BK;
-        splits = ceil_div(K, kchunk);
-        if (splits < 1) { splits = 1; kchunk = K; }
-    } else {
-        split_choice(tiles * batch, tile_slots<BM, BN>(), K, &splits, (tm == 1 || tn == 1) ? 64 : 256);
-        if (splits > 1) {
-            kchunk = ceil_div(ceil_div(K, splits), GEMM_BK) * GEMM_BK;
-            splits = ceil_div(K, kchunk);
+    for (int t = 0; t < 5; t++) {
+        if (!direct && t < 3) continue;                 // unaligned rows: 64 x 64 and 32 x 32 only
+        if (upper && GEMM_TILES[t].bm != GEMM_TILES[t].bn) continue;
+        for (const int s : S) {
+            if (s > 1 && (K / s < 64 || 8 * s * M * N * batch > GEMM_STAGING_MAX)) break;
+            const double c = gemm_cost(GEMM_TILES[t], M, N, K, batch, s, upper, cus);
+            if (c < best) { best = c; *tile = t; *splits = s; }
         }
     }
-    // accumulate in the epilogue when the tiles fit in one round of half the
-    // resident workgroups (the variant's lower occupancy then costs nothing),
-    // or when K is short: the product is then bound by the C traffic, and the
-    // staged path's workspace write and reduction pass would double it
-    if (!upper && splits == 1 && beta != 0.0 && (2 * tiles * batch <= tile_slots<BM, BN>() || K <= 256)) {
-        dim3 grid((unsigned)tiles, 1, (unsigned)batch);
-        ProfScope prof(c, XR_K_GEMM_F64, 2.0 * M * N * K * batch, 8.0 * (M * K + K * N + 2 * M * N) * batch);
-        prof.shape(M, N, K, batch, ta, tb);
-#define XR_GEMM_ACC(TA_, TB_)                                                                    \
-    k_dgemm_acc<BM, BN, TA_, TB_><<<grid, GEMM_THREADS, 0, c->stream>>>(M, N, K, alpha, A, lda, sA, \
-                                                                        B, ldb, sB, beta, C, ldc,  \
-                                                                        sC, tm, tn)
-        if (ta && tb) XR_GEMM_ACC(true, true);
-        else if (ta) XR_GEMM_ACC(true, false);
-        else if (tb) XR_GEMM_ACC(false, true);
-        else XR_GEMM_ACC(false, false);
-#undef XR_GEMM_ACC
-        XR_LAUNCH_CHECK(c);
-        return XR_OK;
-    }
+}
+
+// Bytes of staging a product counts as needing when memory is capped: the
+// rule by which xr_gemm_f64_noalloc, a pinned context and one with a memory
+// limit refuse a call.  It is stated in the sizes (K splits toward full rounds of
+// workgroups, and a staged beta over a large output) and not in how the product
+// runs, so a faster split or an epilogue that needs no staging does not
+// change what a caller can rely on.
+static int64_t gemm_refusal_bytes(int64_t M, int64_t N, int64_t K, bool beta, int64_t batch, bool upper) {
+    const int64_t cus = device_cus();
+    auto choice = [&](int64_t units, int64_t slots, int64_t* splits, int64_t kmin) {
+        auto score = [&](int64_t s) {
+            const double rounds = std::ceil((double)(units * s) / (double)slots);
+            const double ideal = (double)units * (double)K / (double)slots;
+            const double t = rounds * ((double)K / (double)s + 32.0);
+            return ideal / t / (1.0 + (s > 1 ? (double)(s + 1) * 46.0 / (double)K : 0.0));
+        };
+        double best = score(1);
+        *splits = 1;
+        if (K < 512 || units >= 4 * slots) return best;
+        const int64_t smax = std::min<int64_t>(std::min<int64_t>(512, std::max<int64_t>(64, 2 * slots / units)), K / kmin);
+        for (int64_t s = 2; s <= smax; s++) {
+            const double e = score(s);
+            if (e > best) { best = e; *splits = s; }
+        }
+        return best;
+    };
+    int64_t bm = 64, bn = 64, per = 4, s = 1;
+    const int64_t big = ceil_div(M, 128) * ceil_div(N, 128) * batch;
+    if (upper) { bm = bn = 128; per = 2; }
+    else if (beta && K <= 64) { bm = bn = 64; }
+    else if (big >= 512 || (M > 64 && N > 64 && choice(big, 2 * cus, &s, 256) >= 0.8)) { bm = bn = 128; per = 2; }
+    else if (big >= 64 && N <= 64 && M > 64) { bm = 128; per = 3; }
+    else if (big >= 64 && M <= 64 && N > 64) { bn = 128; per = 3; }
+    const int64_t tm = ceil_div(M, bm), tn = ceil_div(N, bn), units = tm * tn * batch;
+    choice(units, per * cus, &s, (tm == 1 || tn == 1) ? 64 : 256);
+    if (s > 1) s = ceil_div(K, ceil_div(ceil_div(K, s), GEMM_BK) * GEMM_BK);
+    const bool staged = s > 1 || (beta && !(2 * units <= per * cus || K <= 256));
+    return staged ? 8 * s * batch * M * N : 0;
+}
+
+// One product with an explicit tile and K split (0: unsplit).
+static int launch_cfg(xr_ctx* c, int tile, int64_t splits, int ta, int tb, int64_t M, int64_t N, int64_t K,
+                      double alpha, const double* A, int64_t lda, int64_t sA, const double* B, int64_t ldb,
+                      int64_t sB, double beta, double* C, int64_t ldc, int64_t sC, int64_t batch,
+                      bool upper = false) {
+    const bool direct = gemm_direct(ta, tb, M, N, K, A, lda, sA, B, ldb, sB);
+    if (!direct && tile < 3) tile = 3;
+    int64_t kchunk = K;
     double* Cw = C;
-    int64_t ldw = ldc, sCw = sC, sSplit = 0;
-    double aw = alpha, bw = beta;
-    const bool staged = splits > 1 || beta != 0.0;
-    if (staged) {
-        Cw = (double*)xr_workspace(c, 50, splits * batch * M * N * sizeof(double));
-        if (!Cw) return xr_fail(c, XR_ENOMEM, "workspace (split-K)");
-        ldw = N;
-        sCw = M * N;
-        sSplit = batch * M * N;
-        aw = 1.0;
-        bw = 0.0;
+    if (splits > 1) {
+        const int64_t unit = tile == 4 ? 32 : GEMM_BK;
+        kchunk = ceil_div(ceil_div(K, splits), unit) * unit;
+        splits = ceil_div(K, kchunk);
     }
+    if (splits < 1) splits = 1;
+    if (splits > 1) {
+        const int64_t need = splits * batch * M * N * (int64_t)sizeof(double);
+        Cw = (double*)xr_workspace(c, 50, need);
+        if (!Cw) {             // no room for the partial tiles: unsplit (gemm_admit has let the call through)
+            c->pin_blocked = c->noalloc_blocked = false;
+            splits = 1;
+            kchunk = K;
+            Cw = C;
+        }
+    }
+    const GemmTile& T = GEMM_TILES[tile];
+    const int64_t tm = ceil_div(M, T.bm), tn = ceil_div(N, T.bn), tiles = tm * tn;
+    if (tiles > 0x7fffffff || batch > 65535) return xr_fail(c, XR_EUNSUPPORTED, "GEMM grid too large");
+    const bool staged = splits > 1;
+    const int64_t ldw = staged ? N : ldc, sCw = staged ? M * N : sC, sSplit = staged ? batch * M * N : 0;
+    const double aw = staged ? 1.0 : alpha, bw = staged ? 0.0 : beta;
     dim3 grid((unsigned)tiles, (unsigned)splits, (unsigned)batch);
     {
         ProfScope prof(c, XR_K_GEMM_F64, 2.0 * M * N * K * batch, 8.0 * (M * K + K * N + M * N) * batch);
         prof.shape(M, N, K, batch, ta, tb);
-#define XR_GEMM_LAUNCH(TA_, TB_)                                                                 \
-    k_dgemm<BM, BN, TA_, TB_><<<grid, GEMM_THREADS, 0, c->stream>>>(M, N, K, aw, A, lda, sA, B,   \
-                                                                     ldb, sB, bw, Cw, ldw, sCw,   \
-                                                                     tm, tn, kchunk, sSplit, upper ? 1 : 0)
-        if (ta && tb) XR_GEMM_LAUNCH(true, true);
-        else if (ta) XR_GEMM_LAUNCH(true, false);
-        else if (tb) XR_GEMM_LAUNCH(false, true);
-        else XR_GEMM_LAUNCH(false, false);
+#define XR_GEMM_ARGS M, N, K, aw, A, lda, sA, B, ldb, sB, bw, Cw, ldw, sCw
+#define XR_GEMM_LAUNCH(BM_, BN_, TA_, TB_, D_)                                                             \
+    k_dgemm<BM_, BN_, TA_, TB_, D_><<<grid, GEMM_THREADS, 0, c->stream>>>(XR_GEMM_ARGS, tm, tn, kchunk, sSplit, \
+                                                                          upper ? 1 : 0)
+#define XR_GEMM_TRANS(BM_, BN_, D_)                           \
+    if (ta && tb) XR_GEMM_LAUNCH(BM_, BN_, true, true, D_);   \
+    else if (ta) XR_GEMM_LAUNCH(BM_, BN_, true, false, D_);   \
+    else if (tb) XR_GEMM_LAUNCH(BM_, BN_, false, true, D_);   \
+    else XR_GEMM_LAUNCH(BM_, BN_, false, false, D_)
+#define XR_GEMM_SMALL(TA_, TB_)                                                                            \
+    k_dgemm_small<TA_, TB_><<<grid, GEMM_THREADS, 0, c->stream>>>(XR_GEMM_ARGS, (int)tn, kchunk, sSplit, upper ? 1 : 0)
+        if (tile == 4) {
+            if (ta && tb) XR_GEMM_SMALL(true, true);
+            else if (ta) XR_GEMM_SMALL(true, false);
+            else if (tb) XR_GEMM_SMALL(false, true);
+            else XR_GEMM_SMALL(false, false);
+        } else if (!direct) { XR_GEMM_TRANS(64, 64, false); }
+        else if (tile == 0) { XR_GEMM_TRANS(128, 128, true); }
+        else if (tile == 1) { XR_GEMM_TRANS(128, 64, true); }
+        else if (tile == 2) { XR_GEMM_TRANS(64, 128, true); }
+        else { XR_GEMM_TRANS(64, 64, true); }
+#undef XR_GEMM_SMALL
+#undef XR_GEMM_TRANS
 #undef XR_GEMM_LAUNCH
+#undef XR_GEMM_ARGS
         XR_LAUNCH_CHECK(c);
     }
     if (staged) {
         ProfScope prof(c, XR_K_OTHER, 0.0, 8.0 * (splits + 2) * batch * M * N);
-        int rc = splitk_reduce(c, Cw, splits, batch, M, N, alpha, beta, C, ldc, sC);
-        if (rc) return rc;
+        return splitk_reduce(c, Cw, splits, batch, M, N, alpha, beta, C, ldc, sC);
     }
     return XR_OK;
+}
+
+// Refuses a product whose staging (gemm_refusal_bytes) does not fit what
+// the context may hold; remembers the largest that did, as the workspace
+// slot would.
+static int gemm_admit(xr_ctx* c, int64_t bytes) {
+    if (!(c->pins > 0 || c->ws_limit || c->noalloc)) {
+        if (bytes > c->gemm_staging) c->gemm_staging = bytes;
+        return XR_OK;
+    }
+    if (bytes == 0 || (!c->noalloc && bytes <= c->gemm_staging) || xr_workspace_fits(c, 50, bytes)) return XR_OK;
+    c->noalloc_blocked = c->noalloc;
+    c->pin_blocked = !c->noalloc && c->pins > 0;
+    return xr_fail(c, XR_ENOMEM, "workspace (split-K)");
+}
+
+// One product with the configuration chosen for its sizes, kept in a small
+// direct-mapped table of the context (a pure function of the sizes: an entry
+// never goes stale; at most 1024 of them).
+static int launch_chosen(xr_ctx* c, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
+                         int64_t lda, int64_t sA, const double* B, int64_t ldb, int64_t sB, double beta, double* C,
+                         int64_t ldc, int64_t sC, int64_t batch, bool upper = false) {
+    const bool direct = gemm_direct(ta, tb, M, N, K, A, lda, sA, B, ldb, sB);
+    const std::array<int64_t, 5> key{M, N, K, batch, (direct ? 1 : 0) | (upper ? 2 : 0) | (beta != 0.0 ? 4 : 0)};
+    uint64_t h = 0;
+    for (int64_t v : key) h = (h ^ (uint64_t)v) * 0x9E3779B97F4A7C15ull;
+    if (c->gemm_choice.empty()) c->gemm_choice.resize(1024);
+    auto& e = c->gemm_choice[h >> 54];
+    if (e.key != key) {
+        gemm_choose(M, N, K, batch, direct, upper, &e.tile, &e.splits);
+        e.staging = gemm_refusal_bytes(M, N, K, beta != 0.0, batch, upper);
+        e.key = key;
+    }
+    const int rc = gemm_admit(c, e.staging);
+    if (rc) return rc;
+    return launch_cfg(c, e.tile, e.splits, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch,
+                      upper);
 }
 
 // C[i][j] = C[j][i] for i > j: the lower triangle from the upper one (32 x 32
@@ -920,7 +1289,7 @@ __global__ __launch_bounds__(256) void k_mirror_upper(double* __restrict__ C, in
 int xr_dgemm_syrk_tn(xr_ctx* c, int64_t n, int64_t K, double alpha, const double* A, int64_t lda, double* C,
                      int64_t ldc) {
     if (n <= 0) return XR_OK;
-    int rc = launch_tiles<128, 128>(c, 1, 0, n, n, K, alpha, A, lda, 0, A, lda, 0, 0.0, C, ldc, 0, 1, 0, true);
+    int rc = launch_chosen(c, 1, 0, n, n, K, alpha, A, lda, 0, A, lda, 0, 0.0, C, ldc, 0, 1, true);
     if (rc) return rc;
     const int64_t t = ceil_div(n, 32);
     if (t > 65535) return xr_fail(c, XR_EUNSUPPORTED, "matrix too large for the mirror grid");
@@ -935,7 +1304,7 @@ int xr_dgemm_syrk_tn(xr_ctx* c, int64_t n, int64_t K, double alpha, const double
 int xr_dgemm_syrk_nt(xr_ctx* c, int64_t n, int64_t K, double alpha, const double* A, int64_t lda, double* C,
                      int64_t ldc) {
     if (n <= 0) return XR_OK;
-    int rc = launch_tiles<128, 128>(c, 0, 1, n, n, K, alpha, A, lda, 0, A, lda, 0, 0.0, C, ldc, 0, 1, 0, true);
+    int rc = launch_chosen(c, 0, 1, n, n, K, alpha, A, lda, 0, A, lda, 0, 0.0, C, ldc, 0, 1, true);
     if (rc) return rc;
     const int64_t t = ceil_div(n, 32);
     if (t > 65535) return xr_fail(c, XR_EUNSUPPORTED, "matrix too large for the mirror grid");
@@ -956,23 +1325,15 @@ extern "C" int xr_gemm_syrk(xr_ctx* c, int trans, int64_t n, int64_t K, double a
     return trans ? xr_dgemm_syrk_tn(c, n, K, alpha, A, lda, C, ldc) : xr_dgemm_syrk_nt(c, n, K, alpha, A, lda, C, ldc);
 }
 
-// One explicit configuration: tile 0 = 128x128, 1 = 128x64, 2 = 64x128,
-// 3 = 64x64; splits = K splits (0 = the heuristic).
-static int launch_cfg(xr_ctx* c, int tile, int splits, int ta, int tb, int64_t M, int64_t N, int64_t K,
-                      double alpha, const double* A, int64_t lda, int64_t sA, const double* B,
-                      int64_t ldb, int64_t sB, double beta, double* C, int64_t ldc, int64_t sC,
-                      int64_t batch) {
-    switch (tile) {
-    case 0: return launch_tiles<128, 128>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch, splits);
-    case 1: return launch_tiles<128, 64>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch, splits);
-    case 2: return launch_tiles<64, 128>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch, splits);
-    default: return launch_tiles<64, 64>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch, splits);
-    }
+// Shapes xr_dgemm_launch gives to the bandwidth kernels.
+static bool gemm_skinny(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t batch) {
+    if (batch != 1 || N > 8) return false;
+    return (!ta && M >= 1024) || (ta && !tb && M <= 64 && K >= 4096) || (ta && M >= 1024 && K <= 64) ||
+           (!ta && !tb && K >= 4096 && M * (N <= 1 ? 1 : (N <= 2 ? 2 : (N <= 4 ? 4 : 8))) <= 64);
 }
 
-// Chooses the tile shape: the autotuned configuration when the shape has
-// one, else 128x128 when the grid still fills the chip and smaller tiles
-// for skinny or small problems.
+// The bandwidth kernels for tall-skinny shapes, else the autotuned
+// configuration when the shape has one, else the modelled choice.
 int xr_dgemm_launch(xr_ctx* c, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
                     const double* A, int64_t lda, int64_t sA, const double* B, int64_t ldb,
                     int64_t sB, double beta, double* C, int64_t ldc, int64_t sC, int64_t batch) {
@@ -1040,26 +1401,14 @@ int xr_dgemm_launch(xr_ctx* c, int ta, int tb, int64_t M, int64_t N, int64_t K, 
         return XR_OK;
     }
     auto it = c->tune.find(std::array<int64_t, 6>{ta, tb, M, N, K, batch});
-    if (it != c->tune.end())
-        return launch_cfg(c, it->second.first, it->second.second, ta, tb, M, N, K, alpha, A, lda, sA,
-                          B, ldb, sB, beta, C, ldc, sC, batch);
-    // a short-K update of C is a read-modify-write of C: the accumulating
-    // 64 x 64 tiles keep more workgroups (and C loads) in flight
-    if (beta != 0.0 && K <= 64)
-        return launch_tiles<64, 64>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch);
-    // 128 x 128 tiles when they (with a K split where K allows one) fill the
-    // rounds of resident workgroups well; smaller tiles for skinny or
-    // small problems
-    int64_t big = ceil_div(M, 128) * ceil_div(N, 128) * batch, s128 = 1;
-    if (big >= 512 || (M > 64 && N > 64 && split_choice(big, tile_slots<128, 128>(), K, &s128) >= 0.8))
-        return launch_tiles<128, 128>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch);
-    if (big < 64)                  // small products: the most (and K-split) workgroups
-        return launch_tiles<64, 64>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch);
-    if (N <= 64 && M > 64)
-        return launch_tiles<128, 64>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch);
-    if (M <= 64 && N > 64)
-        return launch_tiles<64, 128>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch);
-    return launch_tiles<64, 64>(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch);
+    if (it != c->tune.end()) {
+        const int64_t sp = it->second.second;
+        const int rc = gemm_admit(c, sp > 1 ? 8 * sp * M * N * batch : 0);
+        if (rc) return rc;
+        return launch_cfg(c, it->second.first, sp, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC,
+                          batch);
+    }
+    return launch_chosen(c, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch);
 }
 
 extern "C" int xr_gemm_f64(xr_ctx* c, int transA, int transB, int64_t M, int64_t N, int64_t K,
@@ -1076,11 +1425,11 @@ extern "C" int xr_gemm_f64(xr_ctx* c, int transA, int transB, int64_t M, int64_t
                            sC, batch);
 }
 
-// Launches the problems of one tile shape, XR_GROUP_PROBS per grid (with
-// beta != 0 the accumulating kernel, C_q = alpha op(A_q) op(B_q) + beta C_q;
+// Launches the problems of one tile shape, XR_GROUP_PROBS per grid
+// (C_q = alpha op(A_q) op(B_q) + beta C_q; DIRECT: every problem passes gemm_direct;
 // lower: square products with BM == BN whose grids hold only the tiles on
 // and below the diagonal; kind: the profiler class of the launches).
-template <int BM, int BN>
+template <int BM, int BN, bool DIRECT = true>
 static int launch_grouped(xr_ctx* c, const std::vector<int>& ids, int ta, int tb, const int64_t* M,
                           const int64_t* N, const int64_t* K, double alpha, const double* const* A,
                           const int64_t* lda, const double* const* B, const int64_t* ldb, double* const* C,
@@ -1100,6 +1449,8 @@ static int launch_grouped(xr_ctx* c, const std::vector<int>& ids, int ta, int tb
         double flops = 0.0, bytes = 0.0;
         for (size_t t = l; t < order.size(); t += nl) {
             const int q = order[t];
+            if (DIRECT && !gemm_direct(ta, tb, M[q], N[q], K[q], A[q], lda[q], 0, B[q], ldb[q], 0))
+                return xr_fail(c, XR_EINVAL, "grouped GEMM: rows not 16-byte aligned");
             GemmProb& P = g.p[g.n++];
             P = GemmProb{A[q], B[q], C[q], M[q], N[q], K[q], lda[q], ldb[q], ldc[q],
                          ceil_div(M[q], BM), ceil_div(N[q], BN)};
@@ -1112,21 +1463,37 @@ static int launch_grouped(xr_ctx* c, const std::vector<int>& ids, int ta, int tb
         ProfScope prof(c, kind, flops, bytes);
         prof.shape(g.p[0].M, g.p[0].N, g.p[0].K, g.n, ta, tb);
         const dim3 grid((unsigned)(8 * slots));
-        if (beta != 0.0) {
-            if (ta || !tb) return xr_fail(c, XR_EUNSUPPORTED, "accumulating grouped GEMM: A B^T only");
-            k_dgemm_grouped<BM, BN, false, true, true><<<grid, GEMM_THREADS, 0, c->stream>>>(g);
-        } else if (ta && tb) k_dgemm_grouped<BM, BN, true, true><<<grid, GEMM_THREADS, 0, c->stream>>>(g);
-        else if (ta) k_dgemm_grouped<BM, BN, true, false><<<grid, GEMM_THREADS, 0, c->stream>>>(g);
-        else if (tb) k_dgemm_grouped<BM, BN, false, true><<<grid, GEMM_THREADS, 0, c->stream>>>(g);
-        else k_dgemm_grouped<BM, BN, false, false><<<grid, GEMM_THREADS, 0, c->stream>>>(g);
+#define XR_GROUPED(TA_, TB_) \
+    k_dgemm_grouped<BM, BN, TA_, TB_, DIRECT><<<grid, GEMM_THREADS, 0, c->stream>>>(g)
+        if (ta && tb) XR_GROUPED(true, true);
+        else if (ta) XR_GROUPED(true, false);
+        else if (tb) XR_GROUPED(false, true);
+        else XR_GROUPED(false, false);
+#undef XR_GROUPED
         XR_LAUNCH_CHECK(c);
     }
     return XR_OK;
 }
 
+// launch_grouped for problems of any alignment: those that cannot be loaded
+// in 16-byte chunks run on 64 x 64 tiles.
+template <int BM, int BN>
+static int launch_grouped_any(xr_ctx* c, const std::vector<int>& ids, int ta, int tb, const int64_t* M,
+                              const int64_t* N, const int64_t* K, double alpha, const double* const* A,
+                              const int64_t* lda, const double* const* B, const int64_t* ldb, double* const* C,
+                              const int64_t* ldc, double beta = 0.0, int lower = 0, int kind = XR_K_GEMM_GROUPED) {
+    std::vector<int> even, odd;
+    for (int q : ids)
+        (gemm_direct(ta, tb, M[q], N[q], K[q], A[q], lda[q], 0, B[q], ldb[q], 0) ? even : odd).push_back(q);
+    const int rc = launch_grouped<BM, BN>(c, even, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc, beta, lower, kind);
+    if (rc) return rc;
+    return launch_grouped<64, 64, false>(c, odd, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc, beta, lower, kind);
+}
+
 // C_q = alpha op(A_q) op(B_q) for n independent problems (row-major, the
 // same transposes).  Problems with N > 64 share 128 x 128 tile grids, those
-// with 8 < N <= 64 share 128 x 64 grids (both with M > 64); the rest (the
+// with 8 < N <= 64 share 128 x 64 grids (both with M > 64; 64 x 64 ones when
+// their rows are not 16-byte aligned); the rest (the
 // tall-skinny and small shapes) go to the single-product dispatch, whose
 // bandwidth kernels suit them.  No K split and no beta: every C_q is
 // overwritten.
@@ -1156,9 +1523,9 @@ extern "C" int xr_gemm_grouped(xr_ctx* c, int n, int ta, int tb, const int64_t* 
             if (rc) return rc;
         }
     }
-    int rc = launch_grouped<128, 128>(c, wide, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc);
+    int rc = launch_grouped_any<128, 128>(c, wide, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc);
     if (rc) return rc;
-    return launch_grouped<128, 64>(c, narrow, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc);
+    return launch_grouped_any<128, 64>(c, narrow, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1171,11 +1538,7 @@ extern "C" int xr_gemm_tune(xr_ctx* c, int ta, int tb, int64_t M, int64_t N, int
     if (!c) return XR_EINVAL;
     std::lock_guard<std::mutex> g(c->mu);
     if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || reps <= 0) return xr_fail(c, XR_EINVAL, "bad tune shape");
-    if ((N <= 8 && !ta && batch == 1 && M >= 1024) ||
-        (ta && !tb && batch == 1 && M <= 64 && N <= 8 && K >= 4096) ||
-        (ta && batch == 1 && M >= 1024 && K <= 64 && N <= 8) ||
-        (!ta && !tb && batch == 1 && N <= 8 && K >= 4096 &&
-         M * (N <= 1 ? 1 : (N <= 2 ? 2 : (N <= 4 ? 4 : 8))) <= 64)) {   // bandwidth kernels, not tiled
+    if (gemm_skinny(ta, tb, M, N, K, batch)) {           // bandwidth kernels, not tiled
         if (tile_out) *tile_out = -1;
         if (splits_out) *splits_out = 0;
         if (ms_out) *ms_out = 0.0;
@@ -1213,9 +1576,9 @@ extern "C" int xr_gemm_tune(xr_ctx* c, int ta, int tb, int64_t M, int64_t N, int
         XR_HIP(c, hipEventElapsedTime(&ms, e0, e1));
         best = ms / reps;
     }
-    for (int tile = 0; tile < 4 && !rc; tile++) {
+    for (int tile = 0; tile < 4 && !rc; tile++) {   // the untuned choice covers the 32 x 32 kernel
         for (int sp = 1; sp <= 64; sp *= 2) {
-            if (sp > 1 && K / sp < 256) break;
+            if (sp > 1 && (K / sp < 64 || 8 * sp * M * N * batch > GEMM_STAGING_MAX)) break;
             rc = launch_cfg(c, tile, sp, ta, tb, M, N, K, 1.0, A, lda, sA, B, ldb, sB, 0.0, C, N, sC, batch);
             if (rc) break;
             XR_HIP(c, hipEventRecord(e0, c->stream));

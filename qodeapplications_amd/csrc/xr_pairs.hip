@@ -110,9 +110,9 @@ __global__ __launch_bounds__(256) void k_pair_moves(const WlMove* __restrict__ m
 
 // One output tile per workgroup from the work list: problem, K split and
 // tile coordinates come from the table (XCD-aware order built on the host).
-template <int BM, int BN, bool TA, bool TB>
-__global__ __launch_bounds__(GEMM_THREADS) void k_dgemm_worklist(const WlGemm* __restrict__ probs,
-                                                                 const WlTile* __restrict__ tiles) {
+template <int BM, int BN, bool TA, bool TB, bool DIRECT>
+__global__ __launch_bounds__(GEMM_THREADS, GEMM_WAVES(BM, BN)) void k_dgemm_worklist(
+    const WlGemm* __restrict__ probs, const WlTile* __restrict__ tiles) {
     const WlTile t = tiles[blockIdx.x];
     if (t.prob < 0) return;
     const WlGemm P = probs[t.prob];
@@ -121,8 +121,8 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_dgemm_worklist(const WlGemm* _
     const double* A = P.A + (TA ? kbeg * P.lda : kbeg);
     const double* B = P.B + (TB ? kbeg : kbeg * P.ldb);
     double* C = P.C + (int64_t)t.split * P.split_stride;
-    dgemm_tile<BM, BN, TA, TB>(P.M, P.N, K, P.alpha, A, P.lda, B, P.ldb, C, P.ldc, (int64_t)t.tm * BM,
-                               (int64_t)t.tn * BN);
+    dgemm_tile<BM, BN, TA, TB, DIRECT>(P.M, P.N, K, P.alpha, A, P.lda, B, P.ldb, C, P.ldc, (int64_t)t.tm * BM,
+                                       (int64_t)t.tn * BN);
 }
 
 __global__ __launch_bounds__(256) void k_pair_reduce(const WlReduce* __restrict__ rd) {
@@ -258,6 +258,7 @@ struct Group {
 
 struct GemmLaunch {
     int ta, tb, shape;              // shape 0: 128 x 128, 1: 128 x 64, 2: 64 x 64
+    int direct;                     // every product's rows are 16-byte aligned (gemm_direct; else shape 2)
     int64_t tile_off, ntiles;
     double flops, bytes;            // of the launch's products (profiler records)
 };
@@ -288,7 +289,7 @@ const int64_t SHAPE_BM[3] = {128, 128, 64}, SHAPE_BN[3] = {128, 64, 64};
 
 template <int BM, int BN, bool TA, bool TB>
 int64_t worklist_slots() {
-    static const int64_t r = resident_blocks(reinterpret_cast<const void*>(&k_dgemm_worklist<BM, BN, TA, TB>));
+    static const int64_t r = resident_blocks(reinterpret_cast<const void*>(&k_dgemm_worklist<BM, BN, TA, TB, true>));
     return r;
 }
 
@@ -469,10 +470,12 @@ struct Builder {
             sep[q] = pr[q].two_e && (mode == XR_PREC_SPLIT_F32 ||
                                      (mode == XR_PREC_SPLIT_I8 && xr_i8_pays(pr[q].M, pr[q].N, pr[q].K, 1)));
         // per (ta, tb, shape) class: balance the work over the resident workgroups
-        std::map<std::array<int, 3>, std::vector<int>> classes;
+        std::map<std::array<int, 4>, std::vector<int>> classes;
         for (size_t q = 0; q < pr.size(); q++) {
             if (sep[q]) continue;
-            classes[{pr[q].ta, pr[q].tb, shape_of(pr[q].M, pr[q].N)}].push_back((int)q);
+            const Proto& p = pr[q];
+            const int direct = gemm_direct(p.ta, p.tb, p.M, p.N, p.K, p.A, p.lda, 0, p.B, p.ldb, 0) ? 1 : 0;
+            classes[{p.ta, p.tb, direct ? shape_of(p.M, p.N) : 2, direct}].push_back((int)q);
         }
         for (auto& kv : classes) {
             const int shape = kv.first[2];
@@ -558,7 +561,7 @@ struct Builder {
             }
             size_t len = 0;
             for (auto& l : xl) len = std::max(len, l.size());
-            GemmLaunch L{ta, tb, shape, (int64_t)P.tiles.size(), (int64_t)(8 * len), lfl, lby};
+            GemmLaunch L{ta, tb, shape, kv.first[3], (int64_t)P.tiles.size(), (int64_t)(8 * len), lfl, lby};
             for (size_t j = 0; j < len; j++)
                 for (int x = 0; x < 8; x++)
                     P.tiles.push_back(j < xl[x].size() ? xl[x][j] : WlTile{-1, 0, 0, 0});
@@ -675,12 +678,16 @@ int run_program(xr_ctx* c, const Program& P, const char* dblob) {
             ProfScope prof(c, XR_K_GEMM_WORKLIST, L.flops, L.bytes);
             const dim3 grid((unsigned)L.ntiles);
             const WlTile* t = tiles + L.tile_off;
-#define XR_WL(BM_, BN_)                                                                                   \
-            if (L.tb) k_dgemm_worklist<BM_, BN_, false, true><<<grid, GEMM_THREADS, 0, c->stream>>>(probs, t); \
-            else k_dgemm_worklist<BM_, BN_, false, false><<<grid, GEMM_THREADS, 0, c->stream>>>(probs, t)
-            if (L.shape == 0) { XR_WL(128, 128); }
-            else if (L.shape == 1) { XR_WL(128, 64); }
-            else { XR_WL(64, 64); }
+#define XR_WL(BM_, BN_, D_)                                                                                    \
+            if (L.tb) k_dgemm_worklist<BM_, BN_, false, true, D_><<<grid, GEMM_THREADS, 0, c->stream>>>(probs, t); \
+            else k_dgemm_worklist<BM_, BN_, false, false, D_><<<grid, GEMM_THREADS, 0, c->stream>>>(probs, t)
+            if (L.direct) {
+                if (L.shape == 0) { XR_WL(128, 128, true); }
+                else if (L.shape == 1) { XR_WL(128, 64, true); }
+                else { XR_WL(64, 64, true); }
+            } else {
+                XR_WL(64, 64, false);
+            }
 #undef XR_WL
             XR_LAUNCH_CHECK(c);
         }
