@@ -198,6 +198,14 @@ int xr_monomer_2e_adjoint_keep(xr_ctx *ctx, int n_orbs, int n_core, int n_elec,
                                const double *d_V, const double *d_Ebar, double *d_zbar_bra,
                                double *d_zbar_ket, double *d_Vbar, const double *d_W, int64_t w_len);
 
+/* Fragment FCI sigma vectors: out[v, P] = <P| H |Z_v> (nv x n_configs,
+ * overwritten) for H = sum h_pq p+ q + sum V_pqrs p+ q+ s r over the
+ * fragment's spin orbitals (d_h: dim x dim, d_V: dim^4) and the determinants of
+ * n_elec electrons, nC = C(dim - 2 n_core, n_elec - 2 n_core) of them (replaces
+ * compute_HPsi, general-XRCC/atomic_states/LMO_frozen_Hamiltonian.c:358). */
+int xr_fci_sigma(xr_ctx *ctx, int n_orbs, int n_core, int n_elec, int64_t nv, int64_t nC, const double *d_Z,
+                 const double *d_h, const double *d_V, double *d_out);
+
 /* Strided-batched FP64 GEMM on the matrix cores:
  *   C_b = alpha * op(A_b) * op(B_b) + beta * C_b,  b < batch.
  * transA = 0: A is M x K row-major (A[m*lda+k]); 1: A is K x M (A[k*lda+m]).

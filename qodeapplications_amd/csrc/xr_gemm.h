@@ -14,6 +14,12 @@ int xr_dgemm_syrk_tn(xr_ctx* c, int64_t n, int64_t K, double alpha, const double
 int xr_dgemm_syrk_nt(xr_ctx* c, int64_t n, int64_t K, double alpha, const double* A, int64_t lda, double* C,
                      int64_t ldc);
 
+// C = A B for A (M x K, M = row[n]) cut into row blocks [row[q], row[q + 1]),
+// one grouped launch.  *off == 0 (device): A vanishes outside its diagonal
+// blocks, and each row block runs over its own k range only.
+int xr_dgemm_blocks(xr_ctx* c, int n, const int64_t* row, int64_t K, int64_t N, const double* A, int64_t lda,
+                    const double* B, int64_t ldb, double* C, int64_t ldc, const int* off);
+
 // Split-FP32 product (hi/lo FP32 MFMA, FP64 accumulation) and the
 // precision-switched GEMM used by the two-electron contractions.
 int xr_dgemm_split_launch(xr_ctx* c, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,

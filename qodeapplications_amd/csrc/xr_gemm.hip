@@ -541,6 +541,8 @@ struct GemmProb {
     const double* B;
     double* C;
     int64_t M, N, K, lda, ldb, ldc, tiles_m, tiles_n;
+    const int* off;      // null, or: *off == 0 restricts k to [k0, k1) (even; A and B not transposed)
+    int64_t k0, k1;
 };
 struct GemmGroup {
     int n;
@@ -581,7 +583,14 @@ __global__ __launch_bounds__(GEMM_THREADS, GEMM_WAVES(BM, BN)) void k_dgemm_grou
         tm = first_m + (local % per_group) % gsize;
         tn = (local % per_group) / gsize;
     }
-    dgemm_tile<BM, BN, TA, TB, DIRECT>(P.M, P.N, P.K, g.alpha, P.A, P.lda, P.B, P.ldb, P.C, P.ldc, tm * BM, tn * BN,
+    const double *A = P.A, *B = P.B;
+    int64_t K = P.K;
+    if (!TA && !TB && P.off && *P.off == 0) {
+        A += P.k0;
+        B += P.k0 * P.ldb;
+        K = P.k1 - P.k0;
+    }
+    dgemm_tile<BM, BN, TA, TB, DIRECT>(P.M, P.N, K, g.alpha, A, P.lda, B, P.ldb, P.C, P.ldc, tm * BM, tn * BN,
                                        g.beta);
 }
 
@@ -1433,7 +1442,8 @@ template <int BM, int BN, bool DIRECT = true>
 static int launch_grouped(xr_ctx* c, const std::vector<int>& ids, int ta, int tb, const int64_t* M,
                           const int64_t* N, const int64_t* K, double alpha, const double* const* A,
                           const int64_t* lda, const double* const* B, const int64_t* ldb, double* const* C,
-                          const int64_t* ldc, double beta = 0.0, int lower = 0, int kind = XR_K_GEMM_GROUPED) {
+                          const int64_t* ldc, double beta = 0.0, int lower = 0, int kind = XR_K_GEMM_GROUPED,
+                          const int* off = nullptr, const int64_t* k0 = nullptr, const int64_t* k1 = nullptr) {
     if (lower && BM != BN) return xr_fail(c, XR_EUNSUPPORTED, "lower-triangle grids need square tiles");
     // launches of equal problem counts, problems by decreasing K
     std::vector<int> order(ids);
@@ -1453,7 +1463,7 @@ static int launch_grouped(xr_ctx* c, const std::vector<int>& ids, int ta, int tb
                 return xr_fail(c, XR_EINVAL, "grouped GEMM: rows not 16-byte aligned");
             GemmProb& P = g.p[g.n++];
             P = GemmProb{A[q], B[q], C[q], M[q], N[q], K[q], lda[q], ldb[q], ldc[q],
-                         ceil_div(M[q], BM), ceil_div(N[q], BN)};
+                         ceil_div(M[q], BM), ceil_div(N[q], BN), off, off ? k0[q] : 0, off ? k1[q] : 0};
             if (lower && M[q] != N[q]) return xr_fail(c, XR_EUNSUPPORTED, "lower-triangle grid of a non-square C");
             slots += ceil_div(lower ? P.tiles_m * (P.tiles_m + 1) / 2 : P.tiles_m * P.tiles_n, 8);
             flops += (lower ? 1.0 : 2.0) * M[q] * N[q] * K[q];
@@ -1526,6 +1536,38 @@ extern "C" int xr_gemm_grouped(xr_ctx* c, int n, int ta, int tb, const int64_t* 
     int rc = launch_grouped_any<128, 128>(c, wide, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc);
     if (rc) return rc;
     return launch_grouped_any<128, 64>(c, narrow, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc);
+}
+
+int xr_dgemm_blocks(xr_ctx* c, int n, const int64_t* row, int64_t K, int64_t N, const double* A, int64_t lda,
+                    const double* B, int64_t ldb, double* C, int64_t ldc, const int* off) {
+    std::vector<int> ids;
+    std::vector<int64_t> M(n), Ns(n, N), Ks(n, K), la(n, lda), lb(n, ldb), lc(n, ldc), k0(n), k1(n);
+    std::vector<const double*> As(n), Bs(n, B);
+    std::vector<double*> Cs(n);
+    int64_t most = 0;
+    bool direct = true;
+    for (int q = 0; q < n; q++) {
+        M[q] = row[q + 1] - row[q];
+        As[q] = A + row[q] * lda;
+        Cs[q] = C + row[q] * ldc;
+        k0[q] = row[q] & ~(int64_t)1;                         // whole 16-byte chunks of A's rows
+        k1[q] = std::min<int64_t>(K, (row[q + 1] + 1) & ~(int64_t)1);
+        if (M[q] > 0) ids.push_back(q);
+        most = std::max(most, M[q]);
+        direct = direct && gemm_direct(0, 0, M[q], N, K, As[q], lda, 0, B, ldb, 0);
+    }
+    // every class at most 64 rows: 64 x 64 tiles leave less padding
+    if (direct && most > 64)
+        return launch_grouped<128, 128>(c, ids, 0, 0, M.data(), Ns.data(), Ks.data(), 1.0, As.data(), la.data(),
+                                        Bs.data(), lb.data(), Cs.data(), lc.data(), 0.0, 0, XR_K_GEMM_F64, off,
+                                        k0.data(), k1.data());
+    if (direct)
+        return launch_grouped<64, 64>(c, ids, 0, 0, M.data(), Ns.data(), Ks.data(), 1.0, As.data(), la.data(),
+                                      Bs.data(), lb.data(), Cs.data(), lc.data(), 0.0, 0, XR_K_GEMM_F64, off,
+                                      k0.data(), k1.data());
+    return launch_grouped<64, 64, false>(c, ids, 0, 0, M.data(), Ns.data(), Ks.data(), 1.0, As.data(), la.data(),
+                                         Bs.data(), lb.data(), Cs.data(), lc.data(), 0.0, 0, XR_K_GEMM_F64, off,
+                                         k0.data(), k1.data());
 }
 
 // ---------------------------------------------------------------------------

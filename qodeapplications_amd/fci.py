@@ -11,11 +11,11 @@ orbitals (alpha first), the convention of the XR contractions
 integrals <pq|rs>.  The reference's compute_HPsi takes <pq|rs> itself and
 antisymmetrises inside (:380-440); antisymmetrize() converts.
 
-The sigma runs the factorised density kernels backwards: with the state
-matrix Z on both sides and Ebar = 1, the adjoint of the one-body density
-contracted with h and of the monomer sigma with V gives
-dE/dz_bra[k, P] = sum_Q <P| H |Q> Z[k, Q], i.e. (H Z^T)^T, with the same
-gathers and GEMMs as the forward terms (no determinant-pair loop).
+The sigma is one pass of the monomer two-electron term (xr_fci_sigma): Z
+gathered over the pairs it loses, one product with the antisymmetrised pair
+matrix of V (which carries h too: on N electrons h_pq p+ q is
+h_pq p+ (sum_r r+ r) q / (N - 1)), and the adjoint gather back (no
+determinant-pair loop).
 """
 import numpy as np
 import torch
@@ -54,7 +54,7 @@ class Hamiltonian:
 
     def sigma(self, Z, chunk=64):
         """(H Z^T)^T for Z (n_vec x n_configs) on the device, `chunk` vectors
-        per pass (the one-body adjoint's delta_IJ h weight is chunk^2 dim^2)."""
+        per pass (its scratch is two pair gathers of them)."""
         Z = Z.contiguous()
         if Z.shape[0] <= chunk:
             return self._sigma(Z)
@@ -62,22 +62,10 @@ class Hamiltonian:
 
     def _sigma(self, Z):
         Z = Z.contiguous()
-        nv = Z.shape[0]
-        out = torch.zeros_like(Z)
-        if nv == 0 or self.n_elec == 0:      # H annihilates the vacuum
-            return out
-        ctx = context(self.device.index)
-        dim = 2 * self.n_orbs
-        b = self._block
-        # one-body: Rbar[I, J, p, q] = delta_IJ h[p, q]
-        Rb = torch.zeros(nv, nv, dim, dim, dtype=torch.float64, device=self.device)
-        Rb.view(nv * nv, dim * dim)[::nv + 1] = self.h.reshape(1, -1)
-        ctx.call("xr_density_adjoint", b"ca", self.n_orbs, self.n_core, self.n_elec, nv, self.n_configs, ptr(Z),
-                 nv, self.n_configs, ptr(Z), ptr(Rb), ptr(out), None)
-        if self.n_elec >= 2:
-            Eb = torch.eye(nv, dtype=torch.float64, device=self.device)
-            ctx.call("xr_monomer_2e_adjoint", self.n_orbs, self.n_core, self.n_elec, nv, self.n_configs, ptr(Z),
-                     nv, self.n_configs, ptr(Z), ptr(self.V), ptr(Eb), ptr(out), None, None)
+        out = torch.empty_like(Z)
+        if Z.shape[0]:
+            context(self.device.index).call("xr_fci_sigma", self.n_orbs, self.n_core, self.n_elec, Z.shape[0],
+                                            self.n_configs, ptr(Z), ptr(self.h), ptr(self.V), ptr(out))
         return out
 
     def diagonal(self):

@@ -1,0 +1,102 @@
+"""The pair-matrix product in spin-class order: integrals that conserve the
+spin projection (its blocks alone are multiplied) and integrals that do not
+(the whole matrix), with even and odd numbers of pairs and of vectors, against the
+4-index density contracted with V in torch; and the FCI sigma vectors
+against the one- and two-body adjoints they replace.
+
+Tolerances: the sums have at most dim^4 terms of size |V| |rho|; both sides
+round each within a few hundred units of u = 2^-53 of the absolute sum."""
+import numpy as np
+import pytest
+import torch
+
+from qodeapplications_amd import density as D
+from qodeapplications_amd import synthetic as syn
+from qodeapplications_amd._lib import context, ptr
+from qodeapplications_amd.fci import Hamiltonian
+
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -53
+
+
+def _integrals(n_orbs, seed, mix):
+    rng = np.random.default_rng(seed)
+    I = syn.FragmentBlocked([n_orbs], syn.spatial_h(n_orbs, rng), syn.spatial_V(n_orbs, rng))
+    h, V = I.block("T", (0, 0)), I.block("V", (0, 0, 0, 0)).copy()
+    if mix:      # no spin symmetry, no index symmetry
+        V += 0.1 * rng.standard_normal(V.shape)
+    return h, V
+
+
+@pytest.mark.parametrize("mix", [False, True])
+@pytest.mark.parametrize("n_orbs,n_elec,nI,nJ", [(13, 5, 2, 2), (13, 5, 3, 1), (12, 5, 2, 3), (18, 4, 3, 3), (5, 3, 4, 3)])
+def test_monomer_2e_with_and_without_spin_classes(n_orbs, n_elec, nI, nJ, mix):
+    rng = np.random.default_rng(n_orbs + n_elec)
+    h, V = _integrals(n_orbs, 3, mix)
+    sk = syn.random_states(n_orbs, n_elec, nJ, rng)
+    kb = D.ChargeBlock.from_states(sk, n_orbs, 0)
+    bb = kb if nI == nJ else D.ChargeBlock.from_states(syn.random_states(n_orbs, n_elec, nI, rng), n_orbs, 0)
+    E = D.monomer_2e(bb, kb, V)
+    # <p+ q+ s r> = -<p+ q+ r s>: density string ccaa is p+ q+ r s
+    rho = D.density("ccaa", bb, kb)
+    Vt = torch.as_tensor(V, device="cuda").permute(0, 1, 3, 2).contiguous()
+    # <p+ q+ s r> is rho[.., p, q, s, r], so V[p, q, r, s] goes with its last two axes exchanged
+    ref = (rho.reshape(bb.n_states * kb.n_states, -1) @ Vt.reshape(-1, 1)).view(bb.n_states, kb.n_states)
+    mag = (rho.abs().reshape(bb.n_states * kb.n_states, -1) @ Vt.abs().reshape(-1, 1)).view_as(ref)
+    assert bool(((E - ref).abs() <= 400 * U * mag + 1e-15).all()), float((E - ref).abs().max())
+
+
+@pytest.mark.parametrize("mix", [False, True])
+@pytest.mark.parametrize("n_orbs,n_elec,n_core,nv", [(4, 1, 0, 3), (3, 2, 0, 1), (5, 3, 0, 2), (6, 4, 1, 5),
+                                                     (13, 5, 0, 3), (12, 4, 0, 9), (13, 4, 0, 70)])
+def test_sigma_equals_the_adjoints(n_orbs, n_elec, n_core, nv, mix):
+    h, V = _integrals(n_orbs, 7, mix)
+    H = Hamiltonian(n_orbs, n_elec, h, V, n_core)
+    g = torch.Generator(device="cuda").manual_seed(nv)
+    Z = torch.randn(nv, H.n_configs, dtype=torch.float64, device="cuda", generator=g)
+    got = H.sigma(Z)
+    assert torch.equal(got, H.sigma(Z))
+    ref = torch.zeros_like(Z)
+    dim, nc = 2 * n_orbs, H.n_configs
+    Rb = torch.zeros(nv, nv, dim, dim, dtype=torch.float64, device="cuda")
+    Rb.view(nv * nv, dim * dim)[::nv + 1] = H.h.reshape(1, -1)
+    c = context(0)
+    c.call("xr_density_adjoint", b"ca", n_orbs, n_core, n_elec, nv, nc, ptr(Z), nv, nc, ptr(Z), ptr(Rb), ptr(ref), None)
+    if n_elec >= 2:
+        Eb = torch.eye(nv, dtype=torch.float64, device="cuda")
+        c.call("xr_monomer_2e_adjoint", n_orbs, n_core, n_elec, nv, nc, ptr(Z), nv, nc, ptr(Z), ptr(H.V), ptr(Eb),
+               ptr(ref), None, None)
+    # at most ~dim^2 + dim^4 / 4 products of |H| <= max|V| dim^2 and |Z| per element
+    scale = float(H.V.abs().max()) * n_elec ** 2 * dim * float(Z.abs().max()) + float(H.h.abs().max()) * n_elec
+    assert float((got - ref).abs().max()) < 1e-13 * scale * dim
+
+
+def test_adjoint_outputs_on_their_own():
+    # each output of the two adjoints asked for alone equals the one of the full call
+    rng = np.random.default_rng(2)
+    n, ne, nI, nJ = 6, 4, 3, 5
+    h, V = _integrals(n, 11, True)
+    kb = D.ChargeBlock.from_states(syn.random_states(n, ne, nJ, rng), n, 0)
+    bb = D.ChargeBlock.from_states(syn.random_states(n, ne, nI, rng), n, 0)
+    b3 = D.ChargeBlock.from_states(syn.random_states(n, ne - 1, nI, rng), n, 0)
+    c = context(0)
+    Vd = torch.as_tensor(V, device="cuda")
+    Eb = torch.as_tensor(rng.standard_normal((nI, nJ)), device="cuda")
+    args = (n, 0, ne, nI, bb.n_configs, ptr(bb.coeffs), nJ, kb.n_configs, ptr(kb.coeffs), ptr(Vd), ptr(Eb))
+    z = lambda: (torch.zeros_like(bb.coeffs), torch.zeros_like(kb.coeffs), torch.zeros_like(Vd))
+    full = z()
+    c.call("xr_monomer_2e_adjoint", *args, *[ptr(t) for t in full])
+    for k in range(3):
+        one = z()
+        c.call("xr_monomer_2e_adjoint", *args, *[ptr(t) if i == k else None for i, t in enumerate(one)])
+        assert torch.equal(one[k], full[k])
+    dim = 2 * n
+    Rb = torch.as_tensor(rng.standard_normal((nI, nJ, dim)), device="cuda")
+    args = (b"a", n, 0, ne, nI, b3.n_configs, ptr(b3.coeffs), nJ, kb.n_configs, ptr(kb.coeffs), ptr(Rb))
+    z = lambda: (torch.zeros_like(b3.coeffs), torch.zeros_like(kb.coeffs))
+    full = z()
+    c.call("xr_density_adjoint", *args, *[ptr(t) for t in full])
+    for k in range(2):
+        one = z()
+        c.call("xr_density_adjoint", *args, *[ptr(t) if i == k else None for i, t in enumerate(one)])
+        assert torch.equal(one[k], full[k])
