@@ -621,7 +621,7 @@ extern "C" int xr_density(xr_ctx* c, const char* ops, int n_orbs, int n_core, in
 // class, each over its own class's rows of Y when k_veff found no element
 // between classes (on the device: the host does not wait): integrals that
 // conserve the spin projection then cost (2 aa^2 + ab^2) / nU^2 = 0.385 of the dense
-// product (aa, ab pairs of a class).  18 orbitals, 64 states, 5 electrons (630 x 457k x 630): 5.5 -> 2.3 ms.
+// product (aa, ab pairs of a class).  18 orbitals, 64 states, 5 electrons (630 x 457k x 630): 5.5 -> 3.0 ms.
 // Smaller products are bound by launches and run dense in one.
 #define VEFF_CLASS_FLOPS 5e8
 static int veff_product(xr_ctx* c, const double* V, const double* h, double hs, int dim, bool transposed,

@@ -1544,7 +1544,6 @@ int xr_dgemm_blocks(xr_ctx* c, int n, const int64_t* row, int64_t K, int64_t N, 
     std::vector<int64_t> M(n), Ns(n, N), Ks(n, K), la(n, lda), lb(n, ldb), lc(n, ldc), k0(n), k1(n);
     std::vector<const double*> As(n), Bs(n, B);
     std::vector<double*> Cs(n);
-    int64_t most = 0;
     bool direct = true;
     for (int q = 0; q < n; q++) {
         M[q] = row[q + 1] - row[q];
@@ -1553,14 +1552,11 @@ int xr_dgemm_blocks(xr_ctx* c, int n, const int64_t* row, int64_t K, int64_t N, 
         k0[q] = row[q] & ~(int64_t)1;                         // whole 16-byte chunks of A's rows
         k1[q] = std::min<int64_t>(K, (row[q + 1] + 1) & ~(int64_t)1);
         if (M[q] > 0) ids.push_back(q);
-        most = std::max(most, M[q]);
         direct = direct && gemm_direct(0, 0, M[q], N, K, As[q], lda, 0, B, ldb, 0);
     }
-    // every class at most 64 rows: 64 x 64 tiles leave less padding
-    if (direct && most > 64)
-        return launch_grouped<128, 128>(c, ids, 0, 0, M.data(), Ns.data(), Ks.data(), 1.0, As.data(), la.data(),
-                                        Bs.data(), lb.data(), Cs.data(), lc.data(), 0.0, 0, XR_K_GEMM_F64, off,
-                                        k0.data(), k1.data());
+    // 64 x 64 tiles: a block's k range is short (154 or 324 of 630), so a
+    // tile's first loads and its stores are a large part of it, and five tiles a CU
+    // hide them better than two (18 orbitals, 64 states: 3.35 ms with 128 x 128, 3.2 with 128 x 64, 3.0)
     if (direct)
         return launch_grouped<64, 64>(c, ids, 0, 0, M.data(), Ns.data(), Ks.data(), 1.0, As.data(), la.data(),
                                       Bs.data(), lb.data(), Cs.data(), lc.data(), 0.0, 0, XR_K_GEMM_F64, off,
