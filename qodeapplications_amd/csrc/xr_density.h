@@ -25,10 +25,8 @@ struct OpPlan {
 int xr_plan_op(const char* ops, OpPlan* p);
 int xr_space_masks(xr_ctx* c, int n_orbs, int n_core, int n_elec, const uint64_t** masks,
                    int64_t* n);
-int xr_transpose(xr_ctx* c, const double* z, int64_t nS, int64_t nC, double* zT);
 int xr_side_table(xr_ctx* c, const SidePlan& sd, const uint64_t* Km, int64_t nK, int n_orbs,
                   int n_core, int32_t** tab);
-int xr_gather(xr_ctx* c, const int32_t* tab, int64_t rows, const double* zT, int64_t nS, double* out);
 int xr_density_impl(xr_ctx* c, const char* ops, int n_orbs, int n_core, int n_elec_ket,
                     int64_t nI, int64_t nP, const double* zbra, int64_t nJ, int64_t nQ,
                     const double* zket, double* out);

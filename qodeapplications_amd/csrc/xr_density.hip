@@ -21,6 +21,7 @@
 #include "xr_common.h"
 #include "xr_gemm.h"
 #include "xr_density.h"
+#include <algorithm>
 
 // ---------------------------------------------------------------------------
 // operator plans
@@ -179,20 +180,22 @@ __global__ void k_side_table(SidePlan sd, const uint64_t* __restrict__ Km, int64
     XR_GRID_STRIDE(i, nK * nT) k_side_table_elem(i, sd, Km, nK, dim, n_orbs, n_core, nT, tab);
 }
 
-// zT[c * nS + s] = z[s * nC + c]
-__global__ void k_transpose(const double* __restrict__ z, int64_t nS, int64_t nC,
-                            double* __restrict__ zT) {
+// zT[c * nS + s] = z[s * nC + c] for the side blockIdx.z picks
+struct TransposeSide { const double* z; double* zT; int64_t nS, nC; };
+__global__ void k_transpose(TransposeSide t0, TransposeSide t1) {
+    const TransposeSide t = blockIdx.z ? t1 : t0;
     __shared__ double tile[32][33];
-    int64_t c0 = (int64_t)blockIdx.x * 32, s0 = (int64_t)blockIdx.y * 32;
-    int tx = threadIdx.x, ty = threadIdx.y;  // 32 x 8
+    const int64_t c0 = (int64_t)blockIdx.x * 32, s0 = (int64_t)blockIdx.y * 32;
+    if (c0 >= t.nC || s0 >= t.nS) return;
+    const int tx = threadIdx.x, ty = threadIdx.y;  // 32 x 8
     for (int j = ty; j < 32; j += 8) {
-        int64_t s = s0 + j, c = c0 + tx;
-        if (s < nS && c < nC) tile[j][tx] = z[s * nC + c];
+        const int64_t s = s0 + j, c = c0 + tx;
+        if (s < t.nS && c < t.nC) tile[j][tx] = t.z[s * t.nC + c];
     }
     __syncthreads();
     for (int j = ty; j < 32; j += 8) {
-        int64_t c = c0 + j, s = s0 + tx;
-        if (s < nS && c < nC) zT[c * nS + s] = tile[tx][j];
+        const int64_t c = c0 + j, s = s0 + tx;
+        if (s < t.nS && c < t.nC) t.zT[c * t.nS + s] = tile[tx][j];
     }
 }
 
@@ -204,34 +207,41 @@ __global__ void k_transpose(const double* __restrict__ z, int64_t nS, int64_t nC
 // source rows, then all are stored.  Bound by HBM writes: with one set in
 // flight (one dependent table and row load per store) it wrote 2.0 TB/s on
 // 630 x 7140 rows of 64 states.
+// blockIdx.y picks the side: both factors of a density in one launch.  Element
+// (configuration c, state s) of the coefficients is z[c * sC + s * sS].
 #define GATHER_ROWS 4
+struct GatherSide {
+    const int32_t* tab;
+    const double* z;
+    double* out;
+    int64_t rows, nS, sC, sS;
+};
 template <int SP>
-__global__ __launch_bounds__(256) void k_gather_rows(const int32_t* __restrict__ tab, int64_t rows,
-                                                     const double* __restrict__ zT, int64_t nS,
-                                                     double* __restrict__ out) {
+__global__ __launch_bounds__(256) void k_gather_rows(GatherSide g0, GatherSide g1) {
     constexpr int RPW = 64 / SP;                 // rows per wave and set
+    const GatherSide S = blockIdx.y ? g1 : g0;
     const int lane = threadIdx.x & 63;
     const int sub = lane / SP, s0 = lane % SP;
     const int64_t wave = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (RPW * GATHER_ROWS);
     const int64_t step = (int64_t)gridDim.x * 4 * (RPW * GATHER_ROWS);
-    for (int64_t r0 = wave; r0 < rows; r0 += step) {
+    for (int64_t r0 = wave; r0 < S.rows; r0 += step) {
         int32_t e[GATHER_ROWS];
 #pragma unroll
         for (int g = 0; g < GATHER_ROWS; g++) {
             const int64_t r = r0 + g * RPW + sub;
-            e[g] = r < rows ? tab[r] : 0;
+            e[g] = r < S.rows ? S.tab[r] : 0;
         }
-        for (int64_t s = s0; s < nS; s += SP) {
+        for (int64_t s = s0; s < S.nS; s += SP) {
             double v[GATHER_ROWS];
 #pragma unroll
             for (int g = 0; g < GATHER_ROWS; g++) {
                 const int32_t a = e[g] > 0 ? e[g] : -e[g];
-                v[g] = a ? zT[(int64_t)(a - 1) * nS + s] : 0.0;
+                v[g] = a ? S.z[(int64_t)(a - 1) * S.sC + s * S.sS] : 0.0;
             }
 #pragma unroll
             for (int g = 0; g < GATHER_ROWS; g++) {
                 const int64_t r = r0 + g * RPW + sub;
-                if (r < rows) out[r * nS + s] = e[g] < 0 ? -v[g] : v[g];
+                if (r < S.rows) S.out[r * S.nS + s] = e[g] < 0 ? -v[g] : v[g];
             }
         }
     }
@@ -306,6 +316,56 @@ __global__ __launch_bounds__(256) void k_expand_planes(
     }
 }
 
+// The same expansion turned through LDS: a workgroup takes JB consecutive J
+// of one I and LC consecutive left indices iL, reads the Cc rows of those along J
+// (JB doubles at a time), and writes LC * nR contiguous doubles of each of
+// its planes.  Bound by HBM (8 B written and about 4 read per element); the walk
+// plane by plane above reads Cc one 8-byte element per cache line and counts
+// on L2 for the other planes' share.  caa, 13 orbitals, 32 x 32 states (17576
+// per plane): 100 -> 45 us; 18 orbitals, 64 states: 1.10 -> 0.50 ms.
+// nT sorted right tuples; LDS rows of ntp (odd) doubles.
+template <int JB>
+__global__ __launch_bounds__(256) void k_expand_tile(
+    const double* __restrict__ Cc, int64_t ldc, int64_t nI, int64_t nJ, const int32_t* __restrict__ tabL, int nL,
+    const int32_t* __restrict__ tabR, int nR, int nT, int ntp, int LC, double* __restrict__ out) {
+    extern __shared__ double T[];              // [c][j][t]
+    const int jb = (int)((nJ + JB - 1) / JB);
+    const int64_t I = blockIdx.x / jb, J0 = (int64_t)(blockIdx.x - I * jb) * JB;
+    const int iL0 = blockIdx.y * LC, lc = nL - iL0 < LC ? nL - iL0 : LC;
+    const int tid = threadIdx.x;
+    {
+        const int j = tid % JB, t0 = tid / JB;
+        const int64_t J = J0 + j < nJ ? J0 + j : nJ - 1;
+        for (int c = 0; c < lc; c++) {
+            const int eL = tabL ? tabL[iL0 + c] : 1;
+            if (eL == 0) continue;
+            const double* src = Cc + (int64_t)((eL > 0 ? eL : -eL) - 1) * nI * ldc + I * ldc + J;
+            double* dst = T + (c * JB + j) * ntp;
+#pragma unroll 4
+            for (int t = t0; t < nT; t += 256 / JB) {
+                const double v = src[(int64_t)t * nJ];
+                dst[t] = eL < 0 ? -v : v;
+            }
+        }
+    }
+    __syncthreads();
+    const int len = lc * nR;
+    for (int x = tid; x < len; x += 256) {
+        const int c = x / nR, iR = x - c * nR;
+        const int eL = tabL ? tabL[iL0 + c] : 1, eR = tabR ? tabR[iR] : 1;
+        const int t = (eR > 0 ? eR : -eR) - 1;
+        const double* src = T + c * JB * ntp + (t < 0 ? 0 : t);
+        double* dst = out + (I * nJ + J0) * (int64_t)nL * nR + (int64_t)iL0 * nR + x;
+#pragma unroll
+        for (int j = 0; j < JB; j++) {
+            if (J0 + j >= nJ) break;
+            double v = 0.0;
+            if (eL != 0 && eR != 0) v = eR < 0 ? -src[j * ntp] : src[j * ntp];
+            dst[(int64_t)j * nL * nR] = v;
+        }
+    }
+}
+
 // Veff[u, w] for pairs u = (p<q), w = (a<b) in spin-class order:
 //   V[p,q,b,a] - V[q,p,b,a] - V[p,q,a,b] + V[q,p,a,b]
 // (rows of ld >= nU doubles, the padding zero).  h (or null): adds the
@@ -369,10 +429,43 @@ int xr_space_masks(xr_ctx* c, int n_orbs, int n_core, int n_elec, const uint64_t
     return XR_OK;
 }
 
-int xr_transpose(xr_ctx* c, const double* z, int64_t nS, int64_t nC, double* zT) {
-    if (nS <= 0 || nC <= 0) return XR_OK;
-    dim3 grid((unsigned)ceil_div(nC, 32), (unsigned)ceil_div(nS, 32));
-    k_transpose<<<grid, dim3(32, 8), 0, c->stream>>>(z, nS, nC, zT);
+// Coefficients as a gather reads them: the stored (n_states x n_configs)
+// array, or a copy with the state index fastest.
+struct Coeffs { const double* z; int64_t sC, sS; };
+
+// Up to this many bytes of coefficients are gathered as they are stored, which
+// saves the transposing launch.  With both gathers in one launch, a small product in
+// one piece and the tiled expansion, ca of 9 orbitals, 3 electrons, 8 x 8 states: 21.9 -> 15.6 us
+// (together; not measured apart).
+#define GATHER_DIRECT_BYTES (1 << 20)
+
+// The two blocks' coefficients for a gather, those of size > GATHER_DIRECT_BYTES
+// transposed (one launch; one copy for a block with itself).  A null z is not wanted.
+static int coeffs_for_gather(xr_ctx* c, int slot0, int slot1, int64_t nI, int64_t nP, const double* zbra, int64_t nJ,
+                             int64_t nQ, const double* zket, Coeffs* b, Coeffs* k) {
+    const bool same = zbra && zbra == zket && nI == nJ && nP == nQ;
+    *b = Coeffs{zbra, 1, nP};
+    *k = Coeffs{zket, 1, nQ};
+    TransposeSide t[2];
+    int n = 0;
+    if (zbra && nI * nP * (int64_t)sizeof(double) > GATHER_DIRECT_BYTES) {
+        double* zT = (double*)xr_workspace(c, slot0, nP * nI * sizeof(double));
+        if (!zT) return xr_fail(c, XR_ENOMEM, "workspace (coefficients)");
+        t[n++] = TransposeSide{zbra, zT, nI, nP};
+        *b = Coeffs{zT, nI, 1};
+    }
+    if (same) *k = *b;
+    else if (zket && nJ * nQ * (int64_t)sizeof(double) > GATHER_DIRECT_BYTES) {
+        double* zT = (double*)xr_workspace(c, slot1, nQ * nJ * sizeof(double));
+        if (!zT) return xr_fail(c, XR_ENOMEM, "workspace (coefficients)");
+        t[n++] = TransposeSide{zket, zT, nJ, nQ};
+        *k = Coeffs{zT, nJ, 1};
+    }
+    if (n == 0) return XR_OK;
+    if (n == 1) t[1] = t[0];
+    const dim3 grid((unsigned)ceil_div(std::max(t[0].nC, t[1].nC), 32), (unsigned)ceil_div(std::max(t[0].nS, t[1].nS), 32),
+                    (unsigned)n);
+    k_transpose<<<grid, dim3(32, 8), 0, c->stream>>>(t[0], t[1]);
     XR_LAUNCH_CHECK(c);
     return XR_OK;
 }
@@ -426,25 +519,40 @@ static int pair_table(xr_ctx* c, const SidePlan& sd, const uint64_t* Km, int64_t
     return XR_OK;
 }
 
-// out[r][s] for the `rows` table entries r (k_gather_rows)
-int xr_gather(xr_ctx* c, const int32_t* tab, int64_t rows, const double* zT, int64_t nS, double* out) {
-    const int64_t n = rows * nS;
-    if (n <= 0) return XR_OK;
-    ProfScope prof(c, XR_K_GATHER, 0.0, 8.0 * n + 4.0 * rows);
+// One or two sides gathered (k_gather_rows): in one launch up to
+// GATHER_DIRECT_BYTES of output, where the launch is most of it.  Larger ones go one
+// after the other, since two at once share L2: 67 us apart against 72 together (13
+// orbitals, 32 states), 692 against 745 (18 orbitals, 64 states).
+static int gather(xr_ctx* c, const GatherSide* g, int n) {
+    if (n == 2 && (g[0].rows * g[0].nS + g[1].rows * g[1].nS) * (int64_t)sizeof(double) > GATHER_DIRECT_BYTES) {
+        const int rc = gather(c, g, 1);
+        return rc ? rc : gather(c, g + 1, 1);
+    }
+    int64_t elems = 0, rows = 0, nS = 1;
+    for (int q = 0; q < n; q++) {
+        elems += g[q].rows * g[q].nS;
+        rows = std::max(rows, g[q].rows);
+        nS = std::max(nS, g[q].nS);
+    }
+    if (elems <= 0) return XR_OK;
+    ProfScope prof(c, XR_K_GATHER, 0.0, 8.0 * elems);
     const int sp = nS <= 1 ? 1 : nS <= 2 ? 2 : nS <= 4 ? 4 : nS <= 8 ? 8 : nS <= 16 ? 16 : nS <= 32 ? 32 : 64;
-    const int64_t waves = ceil_div(rows, (64 / sp) * GATHER_ROWS);
-    const unsigned grid = xr_grid(waves * 64);
+    const dim3 grid(xr_grid(ceil_div(rows, (64 / sp) * GATHER_ROWS) * 64), (unsigned)n);
+    const GatherSide &a = g[0], &b = g[n - 1];
     switch (sp) {
-    case 1: k_gather_rows<1><<<grid, 256, 0, c->stream>>>(tab, rows, zT, nS, out); break;
-    case 2: k_gather_rows<2><<<grid, 256, 0, c->stream>>>(tab, rows, zT, nS, out); break;
-    case 4: k_gather_rows<4><<<grid, 256, 0, c->stream>>>(tab, rows, zT, nS, out); break;
-    case 8: k_gather_rows<8><<<grid, 256, 0, c->stream>>>(tab, rows, zT, nS, out); break;
-    case 16: k_gather_rows<16><<<grid, 256, 0, c->stream>>>(tab, rows, zT, nS, out); break;
-    case 32: k_gather_rows<32><<<grid, 256, 0, c->stream>>>(tab, rows, zT, nS, out); break;
-    default: k_gather_rows<64><<<grid, 256, 0, c->stream>>>(tab, rows, zT, nS, out); break;
+    case 1: k_gather_rows<1><<<grid, 256, 0, c->stream>>>(a, b); break;
+    case 2: k_gather_rows<2><<<grid, 256, 0, c->stream>>>(a, b); break;
+    case 4: k_gather_rows<4><<<grid, 256, 0, c->stream>>>(a, b); break;
+    case 8: k_gather_rows<8><<<grid, 256, 0, c->stream>>>(a, b); break;
+    case 16: k_gather_rows<16><<<grid, 256, 0, c->stream>>>(a, b); break;
+    case 32: k_gather_rows<32><<<grid, 256, 0, c->stream>>>(a, b); break;
+    default: k_gather_rows<64><<<grid, 256, 0, c->stream>>>(a, b); break;
     }
     XR_LAUNCH_CHECK(c);
     return XR_OK;
+}
+static GatherSide gather_side(const int32_t* tab, int64_t rows, const Coeffs& z, int64_t nS, double* out) {
+    return GatherSide{tab, z.z, out, rows, nS, z.sC, z.sS};
 }
 
 // The signed index table of k indices (k_index_table) depends on (k, dim)
@@ -492,73 +600,73 @@ static int check_spaces(xr_ctx* c, const OpPlan& pl, int n_orbs, int n_core, int
 enum { WS_ZTB = 0, WS_ZTK, WS_OFF, WS_X = 4, WS_Y, WS_C, WS_VE = 9, WS_W };
 enum { WS_GC = 40, WS_XB, WS_YB, WS_ZBT, WS_WB, WS_VEB, WS_GS };
 
-// The two gathered factors of a density: X (nK x nLt*nI) from the bra
-// coefficients and Y (nK x nT*nJ) from the ket coefficients, over the K
-// space that sits between L and R: the bra space when there is no L, the
-// ket space when there is no R (then X or Y is just the transposed
-// coefficients), else every determinant with n_ket - |R| electrons.
+// The two factors of a density: X (nK x nLt*nI) from the bra coefficients
+// and Y (nK x nT*nJ) from the ket coefficients, over the K space that sits
+// between L and R: the bra space when there is no L, the ket space when there
+// is no R, else every determinant with n_ket - |R| electrons.  Without L
+// (R) the factor is the transpose of the coefficients as they are stored: xT
+// (yT) says that X (Y) points at those, nI x nK (nJ x nK) with rows of ldx (ldy).
 struct Factors {
     const uint64_t* Km = nullptr;
     int64_t nK = 0, nLt = 1, nT = 1;
     int kspace_core = 0;
     const double* X = nullptr;
     const double* Y = nullptr;
+    int xT = 0, yT = 0;
+    int64_t ldx = 0, ldy = 0;
 };
-
-// Both blocks' coefficients with the state index fastest (one copy for a
-// block with itself).
-static int transposed(xr_ctx* c, int64_t nI, int64_t nP, const double* zbra, int64_t nJ, int64_t nQ,
-                      const double* zket, double** zTb, double** zTk) {
-    const bool same = zbra == zket && nI == nJ && nP == nQ;
-    *zTb = (double*)xr_workspace(c, WS_ZTB, nP * nI * sizeof(double));
-    *zTk = same ? *zTb : (double*)xr_workspace(c, WS_ZTK, nQ * nJ * sizeof(double));
-    if (!*zTb || !*zTk) return xr_fail(c, XR_ENOMEM, "workspace (coefficients)");
-    const int rc = xr_transpose(c, zbra, nI, nP, *zTb);
-    return rc || same ? rc : xr_transpose(c, zket, nJ, nQ, *zTk);
-}
 
 static int prepare_factors(xr_ctx* c, const OpPlan& pl, int n_orbs, int n_core, int n_elec_ket,
                            int nb, int64_t nI, int64_t nP, const double* zbra, int64_t nJ,
                            int64_t nQ, const double* zket, Factors* f) {
     const int dim = 2 * n_orbs;
     int rc;
-    double *zTb = nullptr, *zTk = nullptr;
-    if ((rc = transposed(c, nI, nP, zbra, nJ, nQ, zket, &zTb, &zTk))) return rc;
     f->nT = pl.R.k ? h_binom(dim, pl.R.k) : 1;
     f->nLt = pl.L.k ? h_binom(dim, pl.L.k) : 1;
+    f->ldx = f->nLt * nI;
+    f->ldy = f->nT * nJ;
     if (!pl.L.k) {
         if ((rc = xr_space_masks(c, n_orbs, n_core, nb, &f->Km, &f->nK))) return rc;
-        f->X = zTb;
+        f->X = zbra;
+        f->xT = 1;
+        f->ldx = nP;
         f->kspace_core = n_core;
     } else if (!pl.R.k) {
         if ((rc = xr_space_masks(c, n_orbs, n_core, n_elec_ket, &f->Km, &f->nK))) return rc;
-        f->Y = zTk;
+        f->Y = zket;
+        f->yT = 1;
+        f->ldy = nQ;
         f->kspace_core = n_core;
     } else {
         if ((rc = xr_space_masks(c, n_orbs, 0, n_elec_ket - pl.R.k, &f->Km, &f->nK))) return rc;
         f->kspace_core = 0;
     }
-    int32_t* tabL = nullptr;
+    Coeffs cb, ck;
+    if ((rc = coeffs_for_gather(c, WS_ZTB, WS_ZTK, nI, nP, pl.L.k ? zbra : nullptr, nJ, nQ,
+                                pl.R.k ? zket : nullptr, &cb, &ck)))
+        return rc;
+    GatherSide g[2];
+    int n = 0;
+    int32_t *tabL = nullptr, *tabR = nullptr;
     if (pl.L.k) {
         double* Xb = (double*)xr_workspace(c, WS_X, f->nK * f->nLt * nI * sizeof(double));
         if (!Xb) return xr_fail(c, XR_ENOMEM, "workspace (bra gather)");
         if ((rc = xr_side_table(c, pl.L, f->Km, f->nK, n_orbs, n_core, &tabL))) return rc;
-        if ((rc = xr_gather(c, tabL, f->nK * f->nLt, zTb, nI, Xb))) return rc;
+        g[n++] = gather_side(tabL, f->nK * f->nLt, cb, nI, Xb);
         f->X = Xb;
     }
     if (pl.R.k) {
-        int32_t* tabR = nullptr;
         if ((rc = xr_side_table(c, pl.R, f->Km, f->nK, n_orbs, n_core, &tabR))) return rc;
         if (pl.L.k && tabR == tabL && zbra == zket && nI == nJ && nP == nQ) {
             f->Y = f->X;                    // a block with itself through one table: the same factor
         } else {
             double* Yb = (double*)xr_workspace(c, WS_Y, f->nK * f->nT * nJ * sizeof(double));
             if (!Yb) return xr_fail(c, XR_ENOMEM, "workspace (ket gather)");
-            if ((rc = xr_gather(c, tabR, f->nK * f->nT, zTk, nJ, Yb))) return rc;
+            g[n++] = gather_side(tabR, f->nK * f->nT, ck, nJ, Yb);
             f->Y = Yb;
         }
     }
-    return XR_OK;
+    return n ? gather(c, g, n) : XR_OK;
 }
 
 int xr_density_impl(xr_ctx* c, const char* ops, int n_orbs, int n_core, int n_elec_ket,
@@ -581,10 +689,12 @@ int xr_density_impl(xr_ctx* c, const char* ops, int n_orbs, int n_core, int n_el
     const int64_t Mg = f.nLt * nI, Ng = f.nT * nJ;
     double* Cc = (double*)xr_workspace(c, WS_C, Mg * Ng * sizeof(double));
     if (!Cc) return xr_fail(c, XR_ENOMEM, "workspace (compressed density)");
-    if (f.X == f.Y && Mg == Ng) {
-        // a block with itself through one factor: Cc = X^T X is symmetric
+    if (f.X == f.Y && Mg == Ng && Mg > 512) {
+        // a block with itself through one factor: Cc = X^T X is symmetric (a
+        // small one is bound by launches, and the mirror is one more)
         if ((rc = xr_dgemm_syrk_tn(c, Mg, f.nK, 1.0, f.X, Mg, Cc, Ng))) return rc;
-    } else if ((rc = xr_dgemm_launch(c, 1, 0, Mg, Ng, f.nK, 1.0, f.X, Mg, 0, f.Y, Ng, 0, 0.0, Cc, Ng, 0, 1))) {
+    } else if ((rc = xr_dgemm_launch(c, f.xT ? 0 : 1, f.yT, Mg, Ng, f.nK, 1.0, f.X, f.ldx, 0, f.Y, f.ldy, 0, 0.0, Cc,
+                                     Ng, 0, 1))) {
         return rc;
     }
     int64_t nIL = 1, nIR = 1;
@@ -595,6 +705,29 @@ int xr_density_impl(xr_ctx* c, const char* ops, int n_orbs, int n_core, int n_el
     int64_t total = nI * nJ * nIL * nIR;
     ProfScope prof(c, XR_K_EXPAND, 0.0, 8.0 * total);
     if (nIL * nIR > 0xffffffffLL - 65536LL * 1024) return xr_fail(c, XR_EUNSUPPORTED, "density plane too large");
+    // through LDS where a tile of JB planes and at least one left index fits
+    // in 48 KB (64 KB for JB = 8); triples on the right (nT > 1000) go plane by plane
+    const int ntp = (int)(f.nT | 1);
+    const int JB = nJ > 8 && 16 * ntp * 8 <= (48 << 10) ? 16 : 8;
+    if ((int64_t)JB * ntp * 8 <= (64 << 10) && nIL * nIR < (1LL << 30)) {
+        const int64_t gx = nI * ceil_div(nJ, JB);
+        int64_t lc = std::max<int64_t>(1, (48 << 10) / ((int64_t)JB * ntp * 8));
+        lc = std::min(lc, std::max<int64_t>(1, nIL * gx / 512));     // enough workgroups first
+        lc = std::min(lc, nIL);
+        const int64_t gy = ceil_div(nIL, lc);
+        if (gx <= 0x7fffffffLL && gy <= 65535) {
+            const dim3 grid((unsigned)gx, (unsigned)gy);
+            const size_t lds = (size_t)lc * JB * ntp * 8;
+            if (JB == 16)
+                k_expand_tile<16><<<grid, 256, lds, c->stream>>>(Cc, Ng, nI, nJ, idxL, (int)nIL, idxR, (int)nIR,
+                                                                 (int)f.nT, ntp, (int)lc, out);
+            else
+                k_expand_tile<8><<<grid, 256, lds, c->stream>>>(Cc, Ng, nI, nJ, idxL, (int)nIL, idxR, (int)nIR,
+                                                                (int)f.nT, ntp, (int)lc, out);
+            XR_LAUNCH_CHECK(c);
+            return XR_OK;
+        }
+    }
     const int64_t planes = nI * nJ;
     const int64_t chunks = ceil_div(nIL * nIR, 1024);
     dim3 grid((unsigned)(planes < (1LL << 30) ? planes : (1LL << 30)),
@@ -657,8 +790,8 @@ static int monomer_2e_impl(xr_ctx* c, int n_orbs, int n_core, int n_elec, int64_
     if (nI <= 0 || nJ <= 0) return XR_OK;
     const int dim = 2 * n_orbs;
     if (n_elec < 2) return xr_fill(c, out, nI * nJ, 0.0);
-    double *zTb = nullptr, *zTk = nullptr;
-    if ((rc = transposed(c, nI, nP, zbra, nJ, nQ, zket, &zTb, &zTk))) return rc;
+    Coeffs cb, ck;
+    if ((rc = coeffs_for_gather(c, WS_ZTB, WS_ZTK, nI, nP, zbra, nJ, nQ, zket, &cb, &ck))) return rc;
     const uint64_t* Km = nullptr;
     int64_t nK = 0;
     if ((rc = xr_space_masks(c, n_orbs, 0, n_elec - 2, &Km, &nK))) return rc;
@@ -674,9 +807,10 @@ static int monomer_2e_impl(xr_ctx* c, int n_orbs, int n_core, int n_elec, int64_
     double* W = Wkeep ? Wkeep : (double*)xr_workspace(c, WS_W, nU * nK * nJ * sizeof(double));
     if ((!same && !X) || !Y || !W) return xr_fail(c, XR_ENOMEM, "workspace (sigma)");
     if ((rc = pair_table(c, pl.R, Km, nK, n_orbs, n_core, &tabR))) return rc;
-    if (!same && ((rc = pair_table(c, pl.L, Km, nK, n_orbs, n_core, &tabL)) ||
-                  (rc = xr_gather(c, tabL, nU * nK, zTb, nI, X)))) return rc;   // X[u][K][I]
-    if ((rc = xr_gather(c, tabR, Kp * nK, zTk, nJ, Y))) return rc;              // Y[w][K][J]
+    if (!same && (rc = pair_table(c, pl.L, Km, nK, n_orbs, n_core, &tabL))) return rc;
+    GatherSide g[2] = {gather_side(tabR, Kp * nK, ck, nJ, Y), GatherSide()};     // Y[w][K][J]
+    if (!same) g[1] = gather_side(tabL, nU * nK, cb, nI, X);                     // X[u][K][I]
+    if ((rc = gather(c, g, same ? 1 : 2))) return rc;
     // W[u][K*nJ + J] = sum_w Ve[u,w] Y[w][K*nJ + J]
     if ((rc = veff_product(c, V, nullptr, 0.0, dim, false, Y, nK * nJ, W))) return rc;
     // E[I,J] = sum_{(u,K)} X[(u,K), I] W[(u,K), J]
@@ -955,7 +1089,7 @@ __global__ void k_sym_sum(const double* __restrict__ G, int64_t n, double* __res
 
 static int side_adjoint(xr_ctx* c, const SidePlan& sd, int n_orbs, int n_core, int kspace_core,
                         int n_elec_src, int64_t nK, int64_t nT, const double* Ybar, int64_t nS,
-                        int layout, double* zbar, double* tmpT, bool add = true) {
+                        int layout, double* zbar, bool add = true) {
     const uint64_t* Sm = nullptr;
     int64_t nS_cfg = 0;
     int rc;
@@ -985,6 +1119,8 @@ static int side_adjoint(xr_ctx* c, const SidePlan& sd, int n_orbs, int n_core, i
             k_side_index<3><<<xr_grid(nS_cfg), 256, 0, c->stream>>>(sd, Sm, nS_cfg, n_orbs, kspace_core, nK, nT, layout, nTup, tab);
         XR_LAUNCH_CHECK(c);
     }
+    double* tmpT = (double*)xr_workspace(c, WS_ZBT, n * sizeof(double));
+    if (!tmpT) return xr_fail(c, XR_ENOMEM, "workspace (side adjoint)");
     if (tab) {
         ProfScope prof(c, XR_K_GATHER, 0.0, 8.0 * n + 4.0 * nS_cfg * nTup);
         k_side_adjoint_tab<<<xr_grid(n), 256, 0, c->stream>>>(tab, nS_cfg, nTup, Ybar, nS, tmpT);
@@ -1044,8 +1180,6 @@ static int monomer_2e_adjoint_impl(xr_ctx* c, int n_orbs, int n_core, int n_elec
     if (nI <= 0 || nJ <= 0 || n_elec < 2) return XR_OK;
     if (!zbar_bra && !zbar_ket && !Vbar) return XR_OK;
     const int dim = 2 * n_orbs;
-    double *zTb = nullptr, *zTk = nullptr;
-    if ((rc = transposed(c, nI, nP, zbra, nJ, nQ, zket, &zTb, &zTk))) return rc;
     const uint64_t* Km = nullptr;
     int64_t nK = 0;
     if ((rc = xr_space_masks(c, n_orbs, 0, n_elec - 2, &Km, &nK))) return rc;
@@ -1074,15 +1208,23 @@ static int monomer_2e_adjoint_impl(xr_ctx* c, int n_orbs, int n_core, int n_elec
     double* Ybar = zbar_ket && !mirror ? (double*)xr_workspace(c, WS_YB, szJ) : nullptr;
     double* Wbar = need_wbar ? (double*)xr_workspace(c, WS_WB, szJ) : nullptr;
     double* Veb = Vbar ? (double*)xr_workspace(c, WS_VEB, nU * nU * sizeof(double)) : nullptr;
-    const int64_t nmax = nP * nI > nQ * nJ ? nP * nI : nQ * nJ;
-    double* zbT = (double*)xr_workspace(c, WS_ZBT, nmax * sizeof(double));
     if ((need_wbar && !mirror && !X) || (need_y && !Y) || (need_w && (!W || !Xbar)) ||
-        (zbar_ket && !mirror && !Ybar) || (need_wbar && !Wbar) || (Vbar && !Veb) || !zbT)
+        (zbar_ket && !mirror && !Ybar) || (need_wbar && !Wbar) || (Vbar && !Veb))
         return xr_fail(c, XR_ENOMEM, "workspace (sigma adjoint)");
-    if (X && ((rc = pair_table(c, pl.L, Km, nK, n_orbs, n_core, &tabL)) ||
-              (rc = xr_gather(c, tabL, Kp * nK, zTb, nI, X)))) return rc;      // X[u][K][I]
-    if (Y && ((rc = pair_table(c, pl.R, Km, nK, n_orbs, n_core, &tabR)) ||
-              (rc = xr_gather(c, tabR, Kp * nK, zTk, nJ, Y)))) return rc;      // Y[w][K][J]
+    Coeffs cb, ck;
+    if ((rc = coeffs_for_gather(c, WS_ZTB, WS_ZTK, nI, nP, X ? zbra : nullptr, nJ, nQ, Y ? zket : nullptr, &cb, &ck)))
+        return rc;
+    GatherSide g[2];
+    int ng = 0;
+    if (X) {                                                                   // X[u][K][I]
+        if ((rc = pair_table(c, pl.L, Km, nK, n_orbs, n_core, &tabL))) return rc;
+        g[ng++] = gather_side(tabL, Kp * nK, cb, nI, X);
+    }
+    if (Y) {                                                                   // Y[w][K][J]
+        if ((rc = pair_table(c, pl.R, Km, nK, n_orbs, n_core, &tabR))) return rc;
+        g[ng++] = gather_side(tabR, Kp * nK, ck, nJ, Y);
+    }
+    if (ng && (rc = gather(c, g, ng))) return rc;
     const int64_t KJ = nK * nJ;
     // W = Ve Y (nU x KJ)
     if (need_w && !Wgiven && (rc = veff_product(c, V, nullptr, 0.0, dim, false, Y, KJ, W))) return rc;
@@ -1114,10 +1256,10 @@ static int monomer_2e_adjoint_impl(xr_ctx* c, int n_orbs, int n_core, int n_elec
     if (Ybar) {
         // Ybar = Ve^T Wbar (nU x KJ)
         if ((rc = veff_product(c, V, nullptr, 0.0, dim, true, Wbar, KJ, Ybar))) return rc;
-        if ((rc = side_adjoint(c, pl.R, n_orbs, n_core, 0, n_elec, nK, nU, Ybar, nJ, 2, zbar_ket, zbT)))
+        if ((rc = side_adjoint(c, pl.R, n_orbs, n_core, 0, n_elec, nK, nU, Ybar, nJ, 2, zbar_ket)))
             return rc;
     }
-    if (zbar_bra && (rc = side_adjoint(c, pl.L, n_orbs, n_core, 0, n_elec, nK, nU, Xbar, nI, 2, zbar_bra, zbT)))
+    if (zbar_bra && (rc = side_adjoint(c, pl.L, n_orbs, n_core, 0, n_elec, nK, nU, Xbar, nI, 2, zbar_bra)))
         return rc;
     return XR_OK;
 }
@@ -1125,7 +1267,7 @@ static int monomer_2e_adjoint_impl(xr_ctx* c, int n_orbs, int n_core, int n_elec
 // out[v, P] = <P| H |Z_v> (overwritten) for H = sum h_pq p+ q + sum V_pqrs p+ q+ s r.
 // With n_elec >= 2 the one-body part is carried by the two-body one
 // (k_veff), so a pass is one gather of Z over the pairs it loses, one pair-matrix product and one side
-// adjoint.  13 orbitals, 5 electrons, 21 vectors: 1.86 -> 0.24 ms against the two adjoints it replaces, whose
+// adjoint.  13 orbitals, 5 electrons, 21 vectors: 1.86 -> 0.22 ms against the two adjoints it replaces, whose
 // one-body weight was a dense delta_IJ h over all vector pairs and whose
 // ket-side products were computed and dropped.
 extern "C" int xr_fci_sigma(xr_ctx* c, int n_orbs, int n_core, int n_elec, int64_t nv, int64_t nC, const double* Z,
@@ -1146,17 +1288,17 @@ extern "C" int xr_fci_sigma(xr_ctx* c, int n_orbs, int n_core, int n_elec, int64
     int64_t nK = 0;
     if ((rc = xr_space_masks(c, n_orbs, 0, n_elec - 2, &Km, &nK))) return rc;
     const int64_t nU = h_binom(dim, 2), Kp = even_up(nU), N = nK * nv;
-    double* zT = (double*)xr_workspace(c, WS_ZTB, nC * nv * sizeof(double));
     double* Y = (double*)xr_workspace(c, WS_Y, Kp * N * sizeof(double));
     double* W = (double*)xr_workspace(c, WS_W, nU * N * sizeof(double));
-    double* zbT = (double*)xr_workspace(c, WS_ZBT, nC * nv * sizeof(double));
-    if (!zT || !Y || !W || !zbT) return xr_fail(c, XR_ENOMEM, "workspace (FCI sigma)");
+    if (!Y || !W) return xr_fail(c, XR_ENOMEM, "workspace (FCI sigma)");
     int32_t* tab = nullptr;
-    if ((rc = xr_transpose(c, Z, nv, nC, zT)) || (rc = pair_table(c, pl.R, Km, nK, n_orbs, n_core, &tab)) ||
-        (rc = xr_gather(c, tab, Kp * nK, zT, nv, Y)) ||
-        (rc = veff_product(c, V, h, 1.0 / (n_elec - 1), dim, false, Y, N, W)))
+    Coeffs cz, none;
+    if ((rc = coeffs_for_gather(c, WS_ZTB, WS_ZTK, nv, nC, Z, 0, 0, nullptr, &cz, &none)) ||
+        (rc = pair_table(c, pl.R, Km, nK, n_orbs, n_core, &tab)))
         return rc;
-    return side_adjoint(c, pl.L, n_orbs, n_core, 0, n_elec, nK, nU, W, nv, 2, out, zbT, false);
+    const GatherSide gs = gather_side(tab, Kp * nK, cz, nv, Y);
+    if ((rc = gather(c, &gs, 1)) || (rc = veff_product(c, V, h, 1.0 / (n_elec - 1), dim, false, Y, N, W))) return rc;
+    return side_adjoint(c, pl.L, n_orbs, n_core, 0, n_elec, nK, nU, W, nv, 2, out, false);
 }
 
 extern "C" int xr_monomer_2e_adjoint(xr_ctx* c, int n_orbs, int n_core, int n_elec, int64_t nI,
@@ -1203,11 +1345,9 @@ extern "C" int xr_density_adjoint(xr_ctx* c, const char* ops, int n_orbs, int n_
     double* Gc = (double*)xr_workspace(c, WS_GC, Mg * Ng * sizeof(double));
     const bool mirror = ops[0] == 'c' && ops[1] == 'a' && ops[2] == 0 && zbra == zket && nI == nJ &&
                         nP == nQ && Mg == Ng && zbar_bra == zbar_ket && zbar_ket && pl.R.k;
-    double* Xbar = zbar_bra && !mirror ? (double*)xr_workspace(c, WS_XB, f.nK * Mg * sizeof(double)) : nullptr;
-    double* Ybar = zbar_ket ? (double*)xr_workspace(c, WS_YB, f.nK * Ng * sizeof(double)) : nullptr;
-    int64_t nmax = nP * nI > nQ * nJ ? nP * nI : nQ * nJ;
-    double* zbT = (double*)xr_workspace(c, WS_ZBT, nmax * sizeof(double));
-    if (!Gc || (zbar_bra && !mirror && !Xbar) || (zbar_ket && !Ybar) || !zbT)
+    double* Xbar = zbar_bra && !mirror && pl.L.k ? (double*)xr_workspace(c, WS_XB, f.nK * Mg * sizeof(double)) : nullptr;
+    double* Ybar = zbar_ket && pl.R.k ? (double*)xr_workspace(c, WS_YB, f.nK * Ng * sizeof(double)) : nullptr;
+    if (!Gc || (zbar_bra && !mirror && pl.L.k && !Xbar) || (zbar_ket && pl.R.k && !Ybar))
         return xr_fail(c, XR_ENOMEM, "workspace (adjoint)");
     {
         int64_t n = Mg * Ng;
@@ -1232,34 +1372,34 @@ extern "C" int xr_density_adjoint(xr_ctx* c, const char* ops, int n_orbs, int n_
         if ((rc = xr_dgemm_launch(c, 0, 0, f.nK, Ng, Mg, 1.0, f.X, Mg, 0, Gs, Ng, 0, 0.0, Ybar, Ng, 0, 1)))
             return rc;
         return side_adjoint(c, pl.R, n_orbs, n_core, f.kspace_core, n_elec_ket, f.nK, f.nT, Ybar, nJ, 0,
-                            zbar_ket, zbT);
+                            zbar_ket);
     }
-    // Ybar = X Gc  (nK x Ng);  Xbar = Y Gc^T  (nK x Mg)
-    if (zbar_ket && (rc = xr_dgemm_launch(c, 0, 0, f.nK, Ng, Mg, 1.0, f.X, Mg, 0, Gc, Ng, 0, 0.0, Ybar, Ng, 0, 1)))
-        return rc;
-    if (zbar_bra && (rc = xr_dgemm_launch(c, 0, 1, f.nK, Mg, Ng, 1.0, f.Y, Ng, 0, Gc, Ng, 0, 0.0, Xbar, Mg, 0, 1)))
-        return rc;
     if (zbar_ket) {
         if (pl.R.k) {
-            if ((rc = side_adjoint(c, pl.R, n_orbs, n_core, f.kspace_core, n_elec_ket, f.nK, f.nT, Ybar,
-                                   nJ, 0, zbar_ket, zbT)))
+            // Ybar = X Gc  (nK x Ng), then the transpose of the gather
+            if ((rc = xr_dgemm_launch(c, f.xT, 0, f.nK, Ng, Mg, 1.0, f.X, f.ldx, 0, Gc, Ng, 0, 0.0, Ybar, Ng, 0, 1)))
+                return rc;
+            if ((rc = side_adjoint(c, pl.R, n_orbs, n_core, f.kspace_core, n_elec_ket, f.nK, f.nT, Ybar, nJ, 0,
+                                   zbar_ket)))
                 return rc;
         } else {
-            // Y = zket^T, so zbar_ket[J, Q] += Ybar[Q, J]
-            dim3 grid((unsigned)ceil_div(nQ, 32), (unsigned)ceil_div(nJ, 32));
-            k_add_transpose<<<grid, dim3(32, 8), 0, c->stream>>>(Ybar, nJ, nQ, zbar_ket, 1);
-            XR_LAUNCH_CHECK(c);
+            // Y = zket^T: zbar_ket (nJ x nQ) += Gc^T X^T
+            if ((rc = xr_dgemm_launch(c, 1, 1, nJ, nQ, Mg, 1.0, Gc, Ng, 0, f.X, f.ldx, 0, 1.0, zbar_ket, nQ, 0, 1)))
+                return rc;
         }
     }
     if (zbar_bra) {
         if (pl.L.k) {
+            // Xbar = Y Gc^T  (nK x Mg)
+            if ((rc = xr_dgemm_launch(c, f.yT, 1, f.nK, Mg, Ng, 1.0, f.Y, f.ldy, 0, Gc, Ng, 0, 0.0, Xbar, Mg, 0, 1)))
+                return rc;
             if ((rc = side_adjoint(c, pl.L, n_orbs, n_core, f.kspace_core, nb, f.nK, f.nLt, Xbar, nI, 0,
-                                   zbar_bra, zbT)))
+                                   zbar_bra)))
                 return rc;
         } else {
-            dim3 grid((unsigned)ceil_div(nP, 32), (unsigned)ceil_div(nI, 32));
-            k_add_transpose<<<grid, dim3(32, 8), 0, c->stream>>>(Xbar, nI, nP, zbar_bra, 1);
-            XR_LAUNCH_CHECK(c);
+            // X = zbra^T: zbar_bra (nI x nP) += Gc Y^T
+            if ((rc = xr_dgemm_launch(c, 0, 1, nI, nP, Ng, 1.0, Gc, Ng, 0, f.Y, f.ldy, 0, 1.0, zbar_bra, nP, 0, 1)))
+                return rc;
         }
     }
     return XR_OK;
