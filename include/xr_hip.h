@@ -289,6 +289,21 @@ int xr_column_norms(xr_ctx *ctx, int64_t n, int b, const double *d_A, int64_t ld
 int xr_transpose(xr_ctx *ctx, int64_t rows, int64_t cols, const double *d_A, int64_t lda, double *d_B,
                  int64_t ldb);
 
+/* Lanczos with full reorthogonalisation for the lowest root of a dense
+ * symmetric A (n x n, n <= 8192).  xr_lanczos_steps runs steps j0 .. j1-1 of at
+ * most cap (<= n), continuing the call that ended at j0; V (cap x n, row
+ * stride ldv) is the basis and work (4 cap + 128 + 2 n) begins with alpha[cap], beta[cap] and
+ * the parts [128, the first ceil(n / 64) in use] of the next vector's squared norm.
+ * xr_lanczos_root: v = V^T s normalised over the first m basis vectors, its Rayleigh
+ * quotient and residual norm in work[0], work[1].  xr_tridiag_lowest (host
+ * arrays): the lowest pair of the tridiagonal (d, e): out = theta, a norm
+ * bound, |s[m-1]|; scratch[2 m]. */
+int xr_lanczos_steps(xr_ctx *ctx, int64_t n, const double *d_A, int64_t lda, int64_t j0, int64_t j1, int64_t cap,
+                     double *d_V, int64_t ldv, double *d_work);
+int xr_lanczos_root(xr_ctx *ctx, int64_t n, const double *d_A, int64_t lda, int64_t m, int64_t cap,
+                    const double *d_V, int64_t ldv, const double *d_s, double *d_work, double *d_v);
+int xr_tridiag_lowest(int64_t m, const double *d, const double *e, double *out, double *s, double *scratch);
+
 /* The Davidson preconditioner's diagonal of a charge sector in the product
  * eigenbasis, and the pair terms' contribution to it:
  *   xr_sector_diag: for each of ntup tuples q (host arrays: dims[q*nf + m],

@@ -68,6 +68,9 @@ SIGNATURES = {
     "xr_residual": (_I, [_P, _L, _I, _I, _P, _L, _P, _L, _P, _P, _L, _P]),
     "xr_column_norms": (_I, [_P, _L, _I, _P, _L, _P, _I]),
     "xr_transpose": (_I, [_P, _L, _L, _P, _L, _P, _L]),
+    "xr_lanczos_steps": (_I, [_P, _L, _P, _L, _L, _L, _L, _P, _L, _P]),
+    "xr_lanczos_root": (_I, [_P, _L, _P, _L, _L, _L, _P, _L, _P, _P, _P]),
+    "xr_tridiag_lowest": (_I, [_L, _P, _P, _P, _P, _P]),
     "xr_sector_diag": (_I, [_P, _I, _I, _P, _P, _P, _P, _P]),
     "xr_column_dots": (_I, [_P, _L, _L, _P, _L, _P, _L, _P]),
     "xr_spin_blocks": (_I, [_P, _I, _P, _P, _P, _P, _P, _L]),

@@ -319,3 +319,263 @@ extern "C" int xr_column_dots(xr_ctx* c, int64_t rows, int64_t cols, const doubl
     XR_LAUNCH_CHECK(c);
     return XR_OK;
 }
+
+// ---------------------------------------------------------------------------
+// Lanczos with full reorthogonalisation for the lowest root of a dense
+// symmetric A (n x n).  One step is one pass over A and two classical
+// Gram-Schmidt passes over the basis V (one vector per row):
+//   k_lz_matvec   V_j = r / |r|, w = A V_j - |r| V_(j-1)
+//   k_lz_dots     c = V w,  k_lz_update  w -= V^T c        (twice; |w|^2 in parts)
+// Every sum has a fixed order, so a root is the same bits on every run.  Bound by
+// launches for n of some hundreds (A sits in L2) and by A's bytes above; the
+// second pass keeps V orthogonal to rounding, without which the alpha / beta
+// factors of a step would amplify the loss.
+// ---------------------------------------------------------------------------
+#define LZ_COLS 64                     // columns of an update block (and of a norm part)
+#define LZ_MAXPART 128                 // n <= LZ_COLS * LZ_MAXPART
+
+__device__ __forceinline__ double wave_sum64(double v) {
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) v += __shfl_xor(v, s, 64);
+    return v;
+}
+
+// start vector in (-1, 1) from the index (splitmix64's mix), with its norm parts
+__global__ __launch_bounds__(LZ_COLS) void k_lz_start(int64_t n, double* __restrict__ r, double* __restrict__ part) {
+    const int64_t i = (int64_t)blockIdx.x * LZ_COLS + threadIdx.x;
+    uint64_t z = (uint64_t)(i + 1) * 0x9e3779b97f4a7c15ULL;
+    z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ULL;
+    z = (z ^ (z >> 27)) * 0x94d049bb133111ebULL;
+    z ^= z >> 31;
+    const double v = i < n ? (double)(int64_t)z * 0x1p-63 : 0.0;
+    if (i < n) r[i] = v;
+    const double t = wave_sum64(v * v);
+    if (threadIdx.x == 0) part[blockIdx.x] = t;
+}
+
+// one wave a row; every wave adds up the nb norm parts of r by itself
+__global__ __launch_bounds__(256) void k_lz_matvec(int64_t n, const double* __restrict__ A, int64_t lda,
+                                                   const double* __restrict__ r, const double* __restrict__ part,
+                                                   int nb, double* __restrict__ Vj, const double* __restrict__ Vp,
+                                                   double* __restrict__ beta, double* __restrict__ w) {
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= n) return;
+    double sq = 0.0;
+    for (int p = lane; p < nb; p += 64) sq += part[p];
+    const double b = sqrt(wave_sum64(sq)), inv = b > 0.0 ? 1.0 / b : 0.0;
+    const double* a = A + row * lda;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    int64_t i = lane;
+    for (; i + 192 < n; i += 256) {
+        s0 += a[i] * r[i];
+        s1 += a[i + 64] * r[i + 64];
+        s2 += a[i + 128] * r[i + 128];
+        s3 += a[i + 192] * r[i + 192];
+    }
+    for (; i < n; i += 64) s0 += a[i] * r[i];
+    const double s = wave_sum64((s0 + s1) + (s2 + s3));
+    if (lane == 0) {
+        Vj[row] = r[row] * inv;
+        w[row] = s * inv - (Vp ? b * Vp[row] : 0.0);
+        if (row == 0 && beta) *beta = b;
+    }
+}
+
+// c[q] = <V_q, w>, one workgroup a basis vector
+__global__ __launch_bounds__(256) void k_lz_dots(int64_t n, const double* __restrict__ V, int64_t ldv,
+                                                 const double* __restrict__ w, double* __restrict__ out) {
+    __shared__ double red[4];
+    const double* v = V + (int64_t)blockIdx.x * ldv;
+    double s0 = 0.0, s1 = 0.0;
+    int64_t i = threadIdx.x;
+    for (; i + 256 < n; i += 512) {
+        s0 += v[i] * w[i];
+        s1 += v[i + 256] * w[i + 256];
+    }
+    if (i < n) s0 += v[i] * w[i];
+    const double s = wave_sum64(s0 + s1);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// w = base - sum_q c_q V_q (base null: + sum) over 64 columns a workgroup, the
+// vectors dealt to 16 waves.  part: |w|^2 of these columns.  alpha = c[m-1] (+ prev[m-1]).
+__global__ __launch_bounds__(1024) void k_lz_update(int64_t n, const double* __restrict__ V, int64_t ldv, int m,
+                                                    const double* __restrict__ c, const double* base,
+                                                    double* w, double* __restrict__ part,
+                                                    const double* __restrict__ prev, double* __restrict__ alpha) {
+    __shared__ double red[16][LZ_COLS];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t i = (int64_t)blockIdx.x * LZ_COLS + lane;
+    double s = 0.0;
+    if (i < n) {
+#pragma unroll 4
+        for (int q = wv; q < m; q += 16) s += c[q] * V[(int64_t)q * ldv + i];
+    }
+    red[wv][lane] = s;
+    __syncthreads();
+    if (wv == 0) {
+        double t = 0.0;
+#pragma unroll
+        for (int q = 0; q < 16; q++) t += red[q][lane];
+        double v = 0.0;
+        if (i < n) {
+            v = base ? base[i] - t : t;
+            w[i] = v;
+        }
+        if (part) {
+            const double sq = wave_sum64(v * v);
+            if (lane == 0) part[blockIdx.x] = sq;
+        }
+        if (alpha && blockIdx.x == 0 && lane == 0) *alpha = c[m - 1] + prev[m - 1];
+    }
+}
+
+// out = {y.w, |w - (y.w) y|} for |y| = 1; one workgroup
+__global__ __launch_bounds__(256) void k_lz_check(int64_t n, const double* __restrict__ y,
+                                                  const double* __restrict__ w, double* __restrict__ out) {
+    __shared__ double red[256];
+    double s = 0.0;
+    for (int64_t i = threadIdx.x; i < n; i += 256) s += y[i] * w[i];
+    const double th = block_sum256(s, red);
+    s = 0.0;
+    for (int64_t i = threadIdx.x; i < n; i += 256) {
+        const double d = w[i] - th * y[i];
+        s += d * d;
+    }
+    const double rr = block_sum256(s, red);
+    if (threadIdx.x == 0) {
+        out[0] = th;
+        out[1] = sqrt(rr);
+    }
+}
+
+// work: alpha[cap], beta[cap] (beta[j] couples j - 1 and j, beta[0] the start's
+// norm), the norm parts of the next vector [LZ_MAXPART], c, c' [cap each], two vectors [n each]
+struct LzWork { double *alpha, *beta, *part, *c0, *c1, *w[2]; };
+static LzWork lz_work(double* p, int64_t cap, int64_t n) {
+    LzWork k;
+    k.alpha = p;
+    k.beta = p + cap;
+    k.part = p + 2 * cap;
+    k.c0 = k.part + LZ_MAXPART;
+    k.c1 = k.c0 + cap;
+    k.w[0] = k.c1 + cap;
+    k.w[1] = k.w[0] + n;
+    return k;
+}
+static int lz_args(xr_ctx* c, int64_t n, const double* A, int64_t lda, int64_t cap, const double* V, int64_t ldv,
+                   const double* work) {
+    if (n < 1 || n > (int64_t)LZ_COLS * LZ_MAXPART || cap < 1 || cap > n)
+        return xr_fail(c, XR_EUNSUPPORTED, "Lanczos: 1 <= steps <= n <= 8192 expected");
+    if (lda < n || ldv < n) return xr_fail(c, XR_ESHAPE, "row stride below n");
+    if (!A || !V || !work) return xr_fail(c, XR_EINVAL, "null operand");
+    return XR_OK;
+}
+
+extern "C" int xr_lanczos_steps(xr_ctx* c, int64_t n, const double* A, int64_t lda, int64_t j0, int64_t j1,
+                                int64_t cap, double* V, int64_t ldv, double* work) {
+    if (!c) return XR_EINVAL;
+    std::lock_guard<std::mutex> g(c->mu);
+    const int rc = lz_args(c, n, A, lda, cap, V, ldv, work);
+    if (rc) return rc;
+    if (j0 < 0 || j1 < j0 || j1 > cap) return xr_fail(c, XR_EINVAL, "Lanczos: step range");
+    const LzWork k = lz_work(work, cap, n);
+    const int nb = (int)ceil_div(n, LZ_COLS);
+    ProfScope prof(c, XR_K_OTHER, 2.0 * n * n * (j1 - j0), 8.0 * n * n * (j1 - j0));
+    if (j0 == 0) k_lz_start<<<nb, LZ_COLS, 0, c->stream>>>(n, k.w[0], k.part);
+    for (int64_t j = j0; j < j1; j++) {
+        double *r = k.w[j & 1], *w = k.w[(j + 1) & 1];
+        k_lz_matvec<<<(unsigned)ceil_div(n, 4), 256, 0, c->stream>>>(n, A, lda, r, k.part, nb, V + j * ldv,
+                                                                     j ? V + (j - 1) * ldv : nullptr, k.beta + j, w);
+        const unsigned m = (unsigned)(j + 1);
+        k_lz_dots<<<m, 256, 0, c->stream>>>(n, V, ldv, w, k.c0);
+        k_lz_update<<<nb, 1024, 0, c->stream>>>(n, V, ldv, (int)m, k.c0, w, w, nullptr, nullptr, nullptr);
+        k_lz_dots<<<m, 256, 0, c->stream>>>(n, V, ldv, w, k.c1);
+        k_lz_update<<<nb, 1024, 0, c->stream>>>(n, V, ldv, (int)m, k.c1, w, w, k.part, k.c0, k.alpha + j);
+    }
+    XR_LAUNCH_CHECK(c);
+    return XR_OK;
+}
+
+// s (device, m): y = V^T s normalised -> v; {Rayleigh quotient, residual norm} -> work's first two doubles
+extern "C" int xr_lanczos_root(xr_ctx* c, int64_t n, const double* A, int64_t lda, int64_t m, int64_t cap,
+                               const double* V, int64_t ldv, const double* s, double* work, double* v) {
+    if (!c) return XR_EINVAL;
+    std::lock_guard<std::mutex> g(c->mu);
+    const int rc = lz_args(c, n, A, lda, cap, V, ldv, work);
+    if (rc) return rc;
+    if (m < 1 || m > cap) return xr_fail(c, XR_EINVAL, "Lanczos: basis size");
+    if (!s || !v) return xr_fail(c, XR_EINVAL, "null operand");
+    const LzWork k = lz_work(work, cap, n);
+    const int nb = (int)ceil_div(n, LZ_COLS);
+    ProfScope prof(c, XR_K_OTHER, 2.0 * n * n, 8.0 * n * n);
+    k_lz_update<<<nb, 1024, 0, c->stream>>>(n, V, ldv, (int)m, s, nullptr, k.w[0], k.part, nullptr, nullptr);
+    k_lz_matvec<<<(unsigned)ceil_div(n, 4), 256, 0, c->stream>>>(n, A, lda, k.w[0], k.part, nb, v, nullptr, nullptr,
+                                                                 k.w[1]);
+    k_lz_check<<<1, 256, 0, c->stream>>>(n, v, k.w[1], k.alpha);
+    XR_LAUNCH_CHECK(c);
+    return XR_OK;
+}
+
+// Lowest eigenpair of the m x m symmetric tridiagonal (d, e), on the host:
+// Sturm bisection, then the vector from a twisted factorisation (top-down
+// and bottom-up LDL^T of T - theta joined where the pivot is least), which keeps small
+// components accurate; the last one decides convergence.  out: theta, the
+// largest |eigenvalue| bound (Gershgorin), |last component|; s[m] normalised.
+extern "C" int xr_tridiag_lowest(int64_t m, const double* d, const double* e, double* out, double* s, double* scratch) {
+    if (m < 1 || !d || (m > 1 && !e) || !out || !s || !scratch) return XR_EINVAL;
+    double lo = 0.0, hi = 0.0;
+    for (int64_t i = 0; i < m; i++) {
+        const double rad = (i ? fabs(e[i - 1]) : 0.0) + (i + 1 < m ? fabs(e[i]) : 0.0);
+        if (!(fabs(d[i]) + rad <= 1e300)) return XR_EINVAL;           // NaN or infinite
+        lo = i ? fmin(lo, d[i] - rad) : d[i] - rad;
+        hi = i ? fmax(hi, d[i] + rad) : d[i] + rad;
+    }
+    const double nrm = fmax(fabs(lo), fabs(hi)), tiny = fmax(nrm, 1e-280) * 0x1p-106;
+    double a = lo, b = hi;                       // lowest eigenvalue in [a, b]
+    for (int it = 0; it < 128; it++) {
+        const double x = 0.5 * (a + b);
+        if (x <= a || x >= b) break;
+        bool below = false;                      // an eigenvalue under x
+        double q = 1.0;
+        for (int64_t i = 0; i < m && !below; i++) {
+            q = d[i] - x - (i ? e[i - 1] * e[i - 1] / q : 0.0);
+            if (fabs(q) < tiny) q = -tiny;
+            below = q < 0.0;
+        }
+        if (below) b = x; else a = x;
+    }
+    const double th = a;
+    double *p = scratch, *q = scratch + m;       // pivots from the top and from the bottom
+    for (int64_t i = 0; i < m; i++) {
+        p[i] = d[i] - th - (i ? e[i - 1] * e[i - 1] / p[i - 1] : 0.0);
+        if (fabs(p[i]) < tiny) p[i] = tiny;
+    }
+    for (int64_t i = m - 1; i >= 0; i--) {
+        q[i] = d[i] - th - (i + 1 < m ? e[i] * e[i] / q[i + 1] : 0.0);
+        if (fabs(q[i]) < tiny) q[i] = tiny;
+    }
+    int64_t r = 0;
+    double best = 0.0;
+    for (int64_t i = 0; i < m; i++) {
+        const double gam = fabs(p[i] + q[i] - (d[i] - th));
+        if (i == 0 || gam < best) {
+            best = gam;
+            r = i;
+        }
+    }
+    s[r] = 1.0;
+    for (int64_t i = r - 1; i >= 0; i--) s[i] = -e[i] * s[i + 1] / p[i];
+    for (int64_t i = r + 1; i < m; i++) s[i] = -e[i - 1] * s[i - 1] / q[i];
+    double nn = 0.0;
+    for (int64_t i = 0; i < m; i++) nn += s[i] * s[i];
+    nn = 1.0 / sqrt(nn);
+    for (int64_t i = 0; i < m; i++) s[i] *= nn;
+    out[0] = th;
+    out[1] = nrm;
+    out[2] = fabs(s[m - 1]);
+    return XR_OK;
+}

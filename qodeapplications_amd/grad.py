@@ -31,7 +31,7 @@ import torch
 
 from ._lib import context, ptr
 from .density import conjugate
-from .eigen import DENSE_MAX
+from .eigen import DENSE_MAX, lowest_root
 from .gemm import mm as _mm, permute4
 from .xr import precision
 
@@ -126,8 +126,7 @@ class XRAdjoint:
         self.op = op = X.operator()
         if op.n <= DENSE_MAX:
             M = op.dense()
-            w, v = torch.linalg.eigh(0.5 * (M + M.T))
-            w, v = w[:1], v[:, :1]
+            w, v = lowest_root(0.5 * (M + M.T))
         else:
             # the gradient is first order in the eigenvector error: converge
             # the residual well below the energy tolerance

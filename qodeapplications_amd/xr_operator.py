@@ -26,7 +26,7 @@ import numpy as np
 import torch
 
 from ._lib import context, ptr
-from .eigen import davidson, precond_divide, upload
+from .eigen import davidson, lowest_root, precond_divide, upload
 from .gemm import gemm_f64, mm, syrk
 
 
@@ -693,7 +693,8 @@ class XROperator:
             if sp.size <= DENSE_SECTOR:
                 M = torch.empty(sp.size, sp.size, dtype=torch.float64, device=self.device)
                 sp.matvec(torch.eye(sp.size, dtype=torch.float64, device=self.device), M)
-                w, v = torch.linalg.eigh(0.5 * (M + M.T))
+                M = 0.5 * (M + M.T)
+                w, v = lowest_root(M) if kk == 1 else torch.linalg.eigh(M)
                 found += [(float(w[i]), sp, v[:, i]) for i in range(kk)]
                 if self.log is not None:
                     self.log.append((sp.Q, sp.size, [float(w[i]) for i in range(kk)], 0.0, 0, "dense"))
