@@ -10,10 +10,10 @@
 //            copy the density columns the one-electron-transfer product
 //            concatenates                                         1 launch
 //   stage 1  density x permuted-integral products of every job: work-list
-//            FP64 MFMA GEMM, one launch per (transpose, tile) class, long
-//            K split over workgroups                          <= 6 launches
+//            FP64 MFMA GEMM, one launch per (transpose, alignment) class,
+//            long K split over workgroups                     <= 4 launches
 //   reduce   split and multi-term partial products, summed in fixed order
-//   stage 2  the bilinear forms' final products (A B^T)       <= 3 launches
+//   stage 2  the bilinear forms' final products (A B^T)       <= 2 launches
 //   reduce
 //   scatter  every job's block, with its spectator-diagonal vectors and
 //            nuclear constant, into the outputs                   1 launch
@@ -257,8 +257,8 @@ struct Group {
 };
 
 struct GemmLaunch {
-    int ta, tb, shape;              // shape 0: 128 x 128, 1: 128 x 64, 2: 64 x 64
-    int direct;                     // every product's rows are 16-byte aligned (gemm_direct; else shape 2)
+    int ta, tb;
+    int direct;                     // every product's rows are 16-byte aligned (gemm_direct)
     int64_t tile_off, ntiles;
     double flops, bytes;            // of the launch's products (profiler records)
 };
@@ -285,29 +285,19 @@ struct Program {
     size_t o_probs = 0, o_tiles = 0, o_moves = 0, o_red[2] = {0, 0}, o_scat = 0, o_sym = 0, blob_bytes = 0;
 };
 
-const int64_t SHAPE_BM[3] = {128, 128, 64}, SHAPE_BN[3] = {128, 64, 64};
+// One tile shape for every product.  A program's products are many and small
+// (rows and columns of a few hundred, ragged), so smaller tiles waste less of
+// them, fill the chip at the end of a launch, and put classes that were launched apart by
+// shape into one launch.  Three fragments of 9, 13 and 18 orbitals with 16, 32 and 8
+// states, with 128 x 128 (128 x 64, 64 x 64 for narrow ones): 1.25 ms, with 128 x 64 at
+// most: 1.16, now: 1.11; two of 18 orbitals and 24 states 1.37 -> 1.18.  10 and 16
+// orbitals with 7 and 29 states lose: 0.412 -> 0.426.
+constexpr int PAIR_TILE = 64;
 
-template <int BM, int BN, bool TA, bool TB>
+template <bool TB>
 int64_t worklist_slots() {
-    static const int64_t r = resident_blocks(reinterpret_cast<const void*>(&k_dgemm_worklist<BM, BN, TA, TB, true>));
+    static const int64_t r = resident_blocks(reinterpret_cast<const void*>(&k_dgemm_worklist<PAIR_TILE, PAIR_TILE, false, TB, true>));
     return r;
-}
-
-int64_t class_slots(int ta, int tb, int shape) {
-    (void)ta;
-    // resident workgroups depend on the tile shape (LDS, registers), not on
-    // the transposes
-    switch (shape) {
-    case 0: return tb ? worklist_slots<128, 128, false, true>() : worklist_slots<128, 128, false, false>();
-    case 1: return tb ? worklist_slots<128, 64, false, true>() : worklist_slots<128, 64, false, false>();
-    default: return tb ? worklist_slots<64, 64, false, true>() : worklist_slots<64, 64, false, false>();
-    }
-}
-
-int shape_of(int64_t M, int64_t N) {
-    if (M > 64 && N > 64) return 0;
-    if (M > 64) return 1;
-    return 2;
 }
 
 void tile_coords(int64_t local, int64_t tm_n, int64_t tn_n, int64_t* tm, int64_t* tn) {
@@ -469,20 +459,19 @@ struct Builder {
         for (size_t q = 0; q < pr.size(); q++)
             sep[q] = pr[q].two_e && (mode == XR_PREC_SPLIT_F32 ||
                                      (mode == XR_PREC_SPLIT_I8 && xr_i8_pays(pr[q].M, pr[q].N, pr[q].K, 1)));
-        // per (ta, tb, shape) class: balance the work over the resident workgroups
-        std::map<std::array<int, 4>, std::vector<int>> classes;
+        // per (ta, tb, direct) class: balance the work over the resident workgroups
+        std::map<std::array<int, 3>, std::vector<int>> classes;
         for (size_t q = 0; q < pr.size(); q++) {
             if (sep[q]) continue;
             const Proto& p = pr[q];
             const int direct = gemm_direct(p.ta, p.tb, p.M, p.N, p.K, p.A, p.lda, 0, p.B, p.ldb, 0) ? 1 : 0;
-            classes[{p.ta, p.tb, direct ? shape_of(p.M, p.N) : 2, direct}].push_back((int)q);
+            classes[{p.ta, p.tb, direct}].push_back((int)q);
         }
         for (auto& kv : classes) {
-            const int shape = kv.first[2];
-            const int64_t bm = SHAPE_BM[shape], bn = SHAPE_BN[shape];
+            const int64_t bm = PAIR_TILE, bn = PAIR_TILE;
             double work = 0.0;
             for (int q : kv.second) work += (double)ceil_div(pr[q].M, bm) * ceil_div(pr[q].N, bn) * pr[q].K;
-            const double slots = (double)class_slots(kv.first[0], kv.first[1], shape);
+            const double slots = (double)(kv.first[1] ? worklist_slots<true>() : worklist_slots<false>());
             // tiles of at most half the balanced per-workgroup K work (and K
             // chunks of at least 256) keep any one tile from running long
             const double target = std::max(256.0, 0.5 * work / slots);
@@ -529,8 +518,8 @@ struct Builder {
         // tile tables: by class, problems by decreasing K chunk, each
         // problem's tiles in contiguous runs over the 8 XCDs
         for (auto& kv : classes) {
-            const int ta = kv.first[0], tb = kv.first[1], shape = kv.first[2];
-            const int64_t bm = SHAPE_BM[shape], bn = SHAPE_BN[shape];
+            const int ta = kv.first[0], tb = kv.first[1];
+            const int64_t bm = PAIR_TILE, bn = PAIR_TILE;
             std::vector<int> order = kv.second;
             std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return kchunk[a] > kchunk[b]; });
             std::vector<std::vector<WlTile>> xl(8);
@@ -561,7 +550,7 @@ struct Builder {
             }
             size_t len = 0;
             for (auto& l : xl) len = std::max(len, l.size());
-            GemmLaunch L{ta, tb, shape, kv.first[3], (int64_t)P.tiles.size(), (int64_t)(8 * len), lfl, lby};
+            GemmLaunch L{ta, tb, kv.first[2], (int64_t)P.tiles.size(), (int64_t)(8 * len), lfl, lby};
             for (size_t j = 0; j < len; j++)
                 for (int x = 0; x < 8; x++)
                     P.tiles.push_back(j < xl[x].size() ? xl[x][j] : WlTile{-1, 0, 0, 0});
@@ -678,16 +667,11 @@ int run_program(xr_ctx* c, const Program& P, const char* dblob) {
             ProfScope prof(c, XR_K_GEMM_WORKLIST, L.flops, L.bytes);
             const dim3 grid((unsigned)L.ntiles);
             const WlTile* t = tiles + L.tile_off;
-#define XR_WL(BM_, BN_, D_)                                                                                    \
-            if (L.tb) k_dgemm_worklist<BM_, BN_, false, true, D_><<<grid, GEMM_THREADS, 0, c->stream>>>(probs, t); \
-            else k_dgemm_worklist<BM_, BN_, false, false, D_><<<grid, GEMM_THREADS, 0, c->stream>>>(probs, t)
-            if (L.direct) {
-                if (L.shape == 0) { XR_WL(128, 128, true); }
-                else if (L.shape == 1) { XR_WL(128, 64, true); }
-                else { XR_WL(64, 64, true); }
-            } else {
-                XR_WL(64, 64, false);
-            }
+#define XR_WL(D_)                                                                                                 \
+            if (L.tb) k_dgemm_worklist<PAIR_TILE, PAIR_TILE, false, true, D_><<<grid, GEMM_THREADS, 0, c->stream>>>(probs, t); \
+            else k_dgemm_worklist<PAIR_TILE, PAIR_TILE, false, false, D_><<<grid, GEMM_THREADS, 0, c->stream>>>(probs, t)
+            if (L.direct) { XR_WL(true); }
+            else { XR_WL(false); }
 #undef XR_WL
             XR_LAUNCH_CHECK(c);
         }
