@@ -105,3 +105,23 @@ def test_nan_and_inf_stay_in_their_rows():
             C = mm(A, B, transA=ta, transB=tb)
             assert bool(torch.isnan(C[M - 1]).all()) and bool(torch.isinf(C[:M - 1, 0]).all())
             assert torch.equal(C[:M - 1, 1:], torch.full_like(C[:M - 1, 1:], float(K)))
+
+
+@pytest.mark.parametrize("odd", [0, 1])
+@pytest.mark.parametrize("rows", [65, 4096, 4160])
+def test_grouped_on_either_side_of_the_one_launch_rule(rows, odd):
+    # 64 x 64 tiles in all: 2 x 8, 64 x 8 = 512 (one launch) and 65 x 8 = 520 (apart by width)
+    shapes = [(rows, 320 - odd, 130), (rows, 64 - odd, 129 + odd), (rows, 128 - odd, 65)]
+    g = torch.Generator(device="cuda").manual_seed(rows + odd)
+    r = lambda a, b: torch.randn(a, b, dtype=torch.float64, device="cuda", generator=g)
+    As, Bs = [r(m, k) for m, w, k in shapes], [r(k, w) for m, w, k in shapes]
+    Cs = [r(m, w) for m, w, k in shapes]
+    n = len(shapes)
+    import ctypes
+    L = lambda v: (ctypes.c_int64 * n)(*v)
+    P = lambda v: (ctypes.c_void_p * n)(*[t.data_ptr() for t in v])
+    M, N, K = (L([s[i] for s in shapes]) for i in range(3))
+    context(0).call("xr_gemm_grouped", n, 0, 0, M, N, K, 1.0, P(As), K, P(Bs), N, P(Cs), N)
+    for A, B, C in zip(As, Bs, Cs):
+        bound = 2 * (A.shape[1] + 2) * 2.0 ** -53 * (A.abs() @ B.abs())
+        assert bool(((C - A @ B).abs() <= bound).all())
