@@ -324,8 +324,8 @@ extern "C" int xr_column_dots(xr_ctx* c, int64_t rows, int64_t cols, const doubl
 // Lanczos with full reorthogonalisation for the lowest root of a dense
 // symmetric A (n x n).  One step is one pass over A and two classical
 // Gram-Schmidt passes over the basis V (one vector per row):
-//   k_lz_matvec   V_j = r / |r|, w = A V_j - |r| V_(j-1)
-//   k_lz_dots     c = V w,  k_lz_update  w -= V^T c        (twice; |w|^2 in parts)
+//   k_root_matvec   V_j = r / |r|, w = A V_j - |r| V_(j-1)
+//   k_root_dots     c = V w,  k_root_update  w -= V^T c        (twice; |w|^2 in parts)
 // Every sum has a fixed order, so a root is the same bits on every run.  Bound by
 // launches for n of some hundreds (A sits in L2) and by A's bytes above; the
 // second pass keeps V orthogonal to rounding, without which the alpha / beta
@@ -341,7 +341,7 @@ __device__ __forceinline__ double wave_sum64(double v) {
 }
 
 // start vector in (-1, 1) from the index (splitmix64's mix), with its norm parts
-__global__ __launch_bounds__(LZ_COLS) void k_lz_start(int64_t n, double* __restrict__ r, double* __restrict__ part) {
+__global__ __launch_bounds__(LZ_COLS) void k_root_start(int64_t n, double* __restrict__ r, double* __restrict__ part) {
     const int64_t i = (int64_t)blockIdx.x * LZ_COLS + threadIdx.x;
     uint64_t z = (uint64_t)(i + 1) * 0x9e3779b97f4a7c15ULL;
     z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ULL;
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(LZ_COLS) void k_lz_start(int64_t n, double* __restr
 }
 
 // one wave a row; every wave adds up the nb norm parts of r by itself
-__global__ __launch_bounds__(256) void k_lz_matvec(int64_t n, const double* __restrict__ A, int64_t lda,
+__global__ __launch_bounds__(256) void k_root_matvec(int64_t n, const double* __restrict__ A, int64_t lda,
                                                    const double* __restrict__ r, const double* __restrict__ part,
                                                    int nb, double* __restrict__ Vj, const double* __restrict__ Vp,
                                                    double* __restrict__ beta, double* __restrict__ w) {
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(256) void k_lz_matvec(int64_t n, const double* __re
 }
 
 // c[q] = <V_q, w>, one workgroup a basis vector
-__global__ __launch_bounds__(256) void k_lz_dots(int64_t n, const double* __restrict__ V, int64_t ldv,
+__global__ __launch_bounds__(256) void k_root_dots(int64_t n, const double* __restrict__ V, int64_t ldv,
                                                  const double* __restrict__ w, double* __restrict__ out) {
     __shared__ double red[4];
     const double* v = V + (int64_t)blockIdx.x * ldv;
@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256) void k_lz_dots(int64_t n, const double* __rest
 
 // w = base - sum_q c_q V_q (base null: + sum) over 64 columns a workgroup, the
 // vectors dealt to 16 waves.  part: |w|^2 of these columns.  alpha = c[m-1] (+ prev[m-1]).
-__global__ __launch_bounds__(1024) void k_lz_update(int64_t n, const double* __restrict__ V, int64_t ldv, int m,
+__global__ __launch_bounds__(1024) void k_root_update(int64_t n, const double* __restrict__ V, int64_t ldv, int m,
                                                     const double* __restrict__ c, const double* base,
                                                     double* w, double* __restrict__ part,
                                                     const double* __restrict__ prev, double* __restrict__ alpha) {
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(1024) void k_lz_update(int64_t n, const double* __r
 }
 
 // out = {y.w, |w - (y.w) y|} for |y| = 1; one workgroup
-__global__ __launch_bounds__(256) void k_lz_check(int64_t n, const double* __restrict__ y,
+__global__ __launch_bounds__(256) void k_root_check(int64_t n, const double* __restrict__ y,
                                                   const double* __restrict__ w, double* __restrict__ out) {
     __shared__ double red[256];
     double s = 0.0;
@@ -485,16 +485,16 @@ extern "C" int xr_lanczos_steps(xr_ctx* c, int64_t n, const double* A, int64_t l
     const LzWork k = lz_work(work, cap, n);
     const int nb = (int)ceil_div(n, LZ_COLS);
     ProfScope prof(c, XR_K_OTHER, 2.0 * n * n * (j1 - j0), 8.0 * n * n * (j1 - j0));
-    if (j0 == 0) k_lz_start<<<nb, LZ_COLS, 0, c->stream>>>(n, k.w[0], k.part);
+    if (j0 == 0) k_root_start<<<nb, LZ_COLS, 0, c->stream>>>(n, k.w[0], k.part);
     for (int64_t j = j0; j < j1; j++) {
         double *r = k.w[j & 1], *w = k.w[(j + 1) & 1];
-        k_lz_matvec<<<(unsigned)ceil_div(n, 4), 256, 0, c->stream>>>(n, A, lda, r, k.part, nb, V + j * ldv,
+        k_root_matvec<<<(unsigned)ceil_div(n, 4), 256, 0, c->stream>>>(n, A, lda, r, k.part, nb, V + j * ldv,
                                                                      j ? V + (j - 1) * ldv : nullptr, k.beta + j, w);
         const unsigned m = (unsigned)(j + 1);
-        k_lz_dots<<<m, 256, 0, c->stream>>>(n, V, ldv, w, k.c0);
-        k_lz_update<<<nb, 1024, 0, c->stream>>>(n, V, ldv, (int)m, k.c0, w, w, nullptr, nullptr, nullptr);
-        k_lz_dots<<<m, 256, 0, c->stream>>>(n, V, ldv, w, k.c1);
-        k_lz_update<<<nb, 1024, 0, c->stream>>>(n, V, ldv, (int)m, k.c1, w, w, k.part, k.c0, k.alpha + j);
+        k_root_dots<<<m, 256, 0, c->stream>>>(n, V, ldv, w, k.c0);
+        k_root_update<<<nb, 1024, 0, c->stream>>>(n, V, ldv, (int)m, k.c0, w, w, nullptr, nullptr, nullptr);
+        k_root_dots<<<m, 256, 0, c->stream>>>(n, V, ldv, w, k.c1);
+        k_root_update<<<nb, 1024, 0, c->stream>>>(n, V, ldv, (int)m, k.c1, w, w, k.part, k.c0, k.alpha + j);
     }
     XR_LAUNCH_CHECK(c);
     return XR_OK;
@@ -512,10 +512,10 @@ extern "C" int xr_lanczos_root(xr_ctx* c, int64_t n, const double* A, int64_t ld
     const LzWork k = lz_work(work, cap, n);
     const int nb = (int)ceil_div(n, LZ_COLS);
     ProfScope prof(c, XR_K_OTHER, 2.0 * n * n, 8.0 * n * n);
-    k_lz_update<<<nb, 1024, 0, c->stream>>>(n, V, ldv, (int)m, s, nullptr, k.w[0], k.part, nullptr, nullptr);
-    k_lz_matvec<<<(unsigned)ceil_div(n, 4), 256, 0, c->stream>>>(n, A, lda, k.w[0], k.part, nb, v, nullptr, nullptr,
+    k_root_update<<<nb, 1024, 0, c->stream>>>(n, V, ldv, (int)m, s, nullptr, k.w[0], k.part, nullptr, nullptr);
+    k_root_matvec<<<(unsigned)ceil_div(n, 4), 256, 0, c->stream>>>(n, A, lda, k.w[0], k.part, nb, v, nullptr, nullptr,
                                                                  k.w[1]);
-    k_lz_check<<<1, 256, 0, c->stream>>>(n, v, k.w[1], k.alpha);
+    k_root_check<<<1, 256, 0, c->stream>>>(n, v, k.w[1], k.alpha);
     XR_LAUNCH_CHECK(c);
     return XR_OK;
 }
