@@ -202,7 +202,8 @@ int xr_monomer_2e_adjoint_keep(xr_ctx *ctx, int n_orbs, int n_core, int n_elec,
  * overwritten) for H = sum h_pq p+ q + sum V_pqrs p+ q+ s r over the
  * fragment's spin orbitals (d_h: dim x dim, d_V: dim^4) and the determinants of
  * n_elec electrons, nC = C(dim - 2 n_core, n_elec - 2 n_core) of them (replaces
- * compute_HPsi, general-XRCC/atomic_states/LMO_frozen_Hamiltonian.c:358). */
+ * compute_HPsi, general-XRCC/atomic_states/LMO_frozen_Hamiltonian.c:358).  FP64
+ * in every precision mode. */
 int xr_fci_sigma(xr_ctx *ctx, int n_orbs, int n_core, int n_elec, int64_t nv, int64_t nC, const double *d_Z,
                  const double *d_h, const double *d_V, double *d_out);
 
@@ -397,8 +398,9 @@ int xr_gemm_mode(xr_ctx *ctx, int mode, int transA, int transB, int64_t M, int64
 
 /* Selects FP64 (XR_PREC_F64, default), split-FP32 (XR_PREC_SPLIT_F32) or
  * split-int8 (XR_PREC_SPLIT_I8) GEMMs for the two-electron contractions (xr_monomer_2e, xr_dimer_2min2pls,
- * xr_dimer_1min1pls_2e, xr_dimer_ExEx, xr_trimer_*).  Densities, one-electron
- * terms and the eigenproblem stay FP64. */
+ * xr_dimer_1min1pls_2e, xr_dimer_ExEx, xr_trimer_*, their adjoints).  Densities,
+ * one-electron terms, the FCI sigma (xr_fci_sigma, whose one- and two-electron
+ * parts share one product) and the eigenproblem stay FP64. */
 int xr_set_precision(xr_ctx *ctx, int mode);
 
 /* Batched H_contractions.c families.  Each evaluates one reference scalar

@@ -750,6 +750,10 @@ extern "C" int xr_density(xr_ctx* c, const char* ops, int n_orbs, int n_core, in
 // and the product W = Ve Y of the two-electron terms, Y (Kp x N, the pairs
 // in spin-class order, its padding row zero).
 //
+// With h (the FCI sigma) the product is FP64 in every precision mode: the
+// matrix then carries the one-electron term, which the split modes leave
+// in FP64, and which being the larger part would also set the split's grids.
+//
 // In FP64 a product of at least VEFF_CLASS_FLOPS runs one problem per spin
 // class, each over its own class's rows of Y when k_veff found no element
 // between classes (on the device: the host does not wait): integrals that
@@ -764,7 +768,8 @@ static int veff_product(xr_ctx* c, const double* V, const double* h, double hs, 
     double* Ve = (double*)xr_workspace(c, WS_VE, nU * Kp * sizeof(double));
     int* off = (int*)xr_workspace(c, WS_OFF, 256);
     if (!Ve || !off) return xr_fail(c, XR_ENOMEM, "workspace (pair matrix)");
-    const bool classes = c->precision == XR_PREC_F64 && 2.0 * nU * nU * N >= VEFF_CLASS_FLOPS;
+    const bool f64 = h || c->precision == XR_PREC_F64;
+    const bool classes = f64 && 2.0 * nU * nU * N >= VEFF_CLASS_FLOPS;
     if (classes) {
         k_set_int<<<1, 1, 0, c->stream>>>(off, 0);
         XR_LAUNCH_CHECK(c);
@@ -772,7 +777,8 @@ static int veff_product(xr_ctx* c, const double* V, const double* h, double hs, 
     k_veff<<<xr_grid(nU * Kp), 256, 0, c->stream>>>(V, h, hs, dim, nU, Kp, transposed ? 1 : 0, Ve,
                                                    classes ? off : nullptr);
     XR_LAUNCH_CHECK(c);
-    if (!classes) return xr_gemm_2e(c, 0, 0, nU, N, Kp, 1.0, Ve, Kp, 0, Y, N, 0, 0.0, W, N, 0, 1);
+    if (!classes)
+        return (f64 ? xr_dgemm_launch : xr_gemm_2e)(c, 0, 0, nU, N, Kp, 1.0, Ve, Kp, 0, Y, N, 0, 0.0, W, N, 0, 1);
     const int64_t row[4] = {0, aa, aa + n * n, nU};
     return xr_dgemm_blocks(c, 3, row, Kp, N, Ve, Kp, Y, N, W, N, off);
 }

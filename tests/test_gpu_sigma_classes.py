@@ -2,7 +2,7 @@
 spin projection (its blocks alone are multiplied) and integrals that do not
 (the whole matrix), with even and odd numbers of pairs and of vectors, against the
 4-index density contracted with V in torch; and the FCI sigma vectors
-against the one- and two-body adjoints they replace.
+against the one- and two-body adjoints they replace, in every precision mode.
 
 Tolerances: the sums have at most dim^4 terms of size |V| |rho|; both sides
 round each within a few hundred units of u = 2^-53 of the absolute sum."""
@@ -14,6 +14,7 @@ from qodeapplications_amd import density as D
 from qodeapplications_amd import synthetic as syn
 from qodeapplications_amd._lib import context, ptr
 from qodeapplications_amd.fci import Hamiltonian
+from qodeapplications_amd.xr import precision
 
 pytestmark = pytest.mark.gpu
 U = 2.0 ** -53
@@ -69,6 +70,19 @@ def test_sigma_equals_the_adjoints(n_orbs, n_elec, n_core, nv, mix):
     # at most ~dim^2 + dim^4 / 4 products of |H| <= max|V| dim^2 and |Z| per element
     scale = float(H.V.abs().max()) * n_elec ** 2 * dim * float(Z.abs().max()) + float(H.h.abs().max()) * n_elec
     assert float((got - ref).abs().max()) < 1e-13 * scale * dim
+
+
+@pytest.mark.parametrize("mode", ["split_f32", "split_i8"])
+@pytest.mark.parametrize("n_orbs,n_elec,nv", [(4, 1, 3), (5, 3, 2), (13, 5, 20)])
+def test_sigma_is_fp64_in_every_mode(n_orbs, n_elec, nv, mode):
+    # the last is large enough for the split-int8 product (2^33 flops)
+    h, V = _integrals(n_orbs, 7, False)
+    H = Hamiltonian(n_orbs, n_elec, h, V)
+    g = torch.Generator(device="cuda").manual_seed(nv)
+    Z = torch.randn(nv, H.n_configs, dtype=torch.float64, device="cuda", generator=g)
+    want = H.sigma(Z)
+    with precision(mode):
+        assert torch.equal(H.sigma(Z), want)
 
 
 def test_adjoint_outputs_on_their_own():
