@@ -4,8 +4,11 @@ spin projection (its blocks alone are multiplied) and integrals that do not
 4-index density contracted with V in torch; and the FCI sigma vectors
 against the one- and two-body adjoints they replace, in every precision mode.
 
-Tolerances: the sums have at most dim^4 terms of size |V| |rho|; both sides
-round each within a few hundred units of u = 2^-53 of the absolute sum."""
+Tolerances, element by element: the monomer sums have at most dim^4 terms of size
+|V| |rho|; both sides round each within a few hundred units of u = 2^-53 of the
+absolute sum.  A sigma element is a sum over at most dim orbitals, nU pairs and the
+N(N-1)/2 pairs of its determinant, so either side is within their number times u of
+the exact one, times the absolute sum (|h| and |V| on |Z|)."""
 import numpy as np
 import pytest
 import torch
@@ -26,7 +29,34 @@ def _integrals(n_orbs, seed, mix):
     h, V = I.block("T", (0, 0)), I.block("V", (0, 0, 0, 0)).copy()
     if mix:      # no spin symmetry, no index symmetry
         V += 0.1 * rng.standard_normal(V.shape)
+        h = h + 0.1 * rng.standard_normal(h.shape)
     return h, V
+
+
+def _abs_sigma(H, Z):
+    """sum |h_pq| |Z| + sum |V_pqrs| |Z| over the terms of every sigma element:
+    |Z| on the determinants less one orbital (two), times |h| (|V| of the four
+    index orders), gathered back over what each determinant loses."""
+    occ = torch.as_tensor(H.configs, device="cuda")
+    masks = (1 << occ).sum(1)
+    dim, N, Zt = 2 * H.n_orbs, H.n_elec, Z.abs().T.contiguous()
+    V = H.V.abs()
+    A4 = V.permute(0, 1, 3, 2) + V.permute(1, 0, 3, 2) + V + V.permute(1, 0, 2, 3)      # [p, q, a, b]
+    mag = torch.zeros_like(Zt)
+    for k in (1, 2):
+        lost = [(i,) for i in range(N)] if k == 1 else [(i, j) for i in range(N) for j in range(i + 1, N)]
+        if not lost:
+            continue
+        K = torch.stack([masks - sum(1 << occ[:, i] for i in t) for t in lost])
+        uniq, K = torch.unique(K, return_inverse=True)
+        u = torch.stack([occ[:, t[0]] if k == 1 else occ[:, t[0]] * dim + occ[:, t[1]] for t in lost])
+        Y = torch.zeros(dim ** k, len(uniq), Zt.shape[1], dtype=torch.float64, device="cuda")
+        for i in range(len(lost)):
+            Y[u[i], K[i]] = Zt
+        W = ((H.h.abs() if k == 1 else A4.reshape(dim * dim, dim * dim)) @ Y.view(dim ** k, -1)).view_as(Y)
+        for i in range(len(lost)):
+            mag += W[u[i], K[i]]
+    return mag.T
 
 
 @pytest.mark.parametrize("mix", [False, True])
@@ -67,9 +97,9 @@ def test_sigma_equals_the_adjoints(n_orbs, n_elec, n_core, nv, mix):
         Eb = torch.eye(nv, dtype=torch.float64, device="cuda")
         c.call("xr_monomer_2e_adjoint", n_orbs, n_core, n_elec, nv, nc, ptr(Z), nv, nc, ptr(Z), ptr(H.V), ptr(Eb),
                ptr(ref), None, None)
-    # at most ~dim^2 + dim^4 / 4 products of |H| <= max|V| dim^2 and |Z| per element
-    scale = float(H.V.abs().max()) * n_elec ** 2 * dim * float(Z.abs().max()) + float(H.h.abs().max()) * n_elec
-    assert float((got - ref).abs().max()) < 1e-13 * scale * dim
+    terms = dim * (dim - 1) // 2 + dim + n_elec ** 2 + 16
+    bound = 2 * terms * U * _abs_sigma(H, Z) + 1e-300
+    assert bool(((got - ref).abs() <= bound).all()), float(((got - ref).abs() / bound).max())
 
 
 @pytest.mark.parametrize("mode", ["split_f32", "split_i8"])
