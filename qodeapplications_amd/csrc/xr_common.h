@@ -124,7 +124,7 @@ struct xr_ctx {
     // tile and K split chosen for recent product sizes (launch_chosen)
     struct GemmChoice { std::array<int64_t, 5> key{-1, -1, -1, -1, -1}; int tile = 3; int64_t splits = 1, staging = 0; };
     std::vector<GemmChoice> gemm_choice;
-    int64_t gemm_staging = 0;   // largest staging admitted since the last trim (gemm_admit)
+    int64_t gemm_staging = 0;   // largest staging admitted since the last trim, backed by slot 50 (gemm_admit)
     // GEMM autotune table: (ta, tb, M, N, K, batch) -> (tile, splits)
     std::map<std::array<int64_t, 6>, std::pair<int, int>> tune;
     // captured graphs holding the workspace addresses (xr_pin): while > 0 a
@@ -163,7 +163,7 @@ struct ProfScope {
 };
 int xr_hip_check(xr_ctx* c, hipError_t e, const char* what);
 void* xr_workspace(xr_ctx* c, int slot, size_t bytes);
-bool xr_workspace_fits(xr_ctx* c, int slot, size_t bytes);
+size_t xr_workspace_room(xr_ctx* c, int slot);
 int xr_noalloc_init(xr_ctx* c);
 int xr_fill(xr_ctx* c, double* p, int64_t n, double v);
 

@@ -1,5 +1,6 @@
 // Context, errors, workspaces, binomial table, configuration masks and ranks.
 #include "xr_common.h"
+#include <algorithm>
 #include <cstring>
 
 __constant__ uint64_t c_binom[65 * 65];
@@ -27,21 +28,21 @@ int xr_hip_check(xr_ctx* c, hipError_t e, const char* what) {
     return xr_fail(c, e == hipErrorOutOfMemory ? XR_ENOMEM : XR_EHIP, m);
 }
 
-// Returns a device buffer of at least `bytes` for scratch slot `slot`,
-// growing it when needed (the old contents are not kept).
-// Whether xr_workspace would serve `bytes` from this slot as far as the
-// caps go (nothing is allocated).
-bool xr_workspace_fits(xr_ctx* c, int slot, size_t bytes) {
-    if (c->noalloc) return c->scratch && bytes <= c->scratch_bytes;
-    if ((int)c->ws.size() > slot && c->ws[slot] && c->ws_size[slot] >= bytes) return true;
-    if (c->pins > 0) return false;
-    if (!c->ws_limit) return true;
-    size_t total = bytes;
+// Bytes xr_workspace could serve from this slot as far as the caps go
+// (nothing is allocated).
+size_t xr_workspace_room(xr_ctx* c, int slot) {
+    if (c->noalloc) return c->scratch ? c->scratch_bytes : 0;
+    const size_t have = (int)c->ws.size() > slot && c->ws[slot] ? c->ws_size[slot] : 0;
+    if (c->pins > 0) return have;
+    if (!c->ws_limit) return SIZE_MAX;
+    size_t others = 0;
     for (size_t i = 0; i < c->ws_size.size(); i++)
-        if ((int)i != slot) total += c->ws_size[i];
-    return total <= c->ws_limit;
+        if ((int)i != slot) others += c->ws_size[i];
+    return std::max(have, c->ws_limit > others ? c->ws_limit - others : (size_t)0);
 }
 
+// Returns a device buffer of at least `bytes` for scratch slot `slot`,
+// growing it when needed (the old contents are not kept).
 void* xr_workspace(xr_ctx* c, int slot, size_t bytes) {
     if (c->noalloc) {           // a no-allocation call: the static scratch array or nothing
         if (c->scratch && bytes <= c->scratch_bytes) return c->scratch;

@@ -1108,13 +1108,14 @@ static double gemm_cost(const GemmTile& t, int64_t M, int64_t N, int64_t K, int6
     return us;
 }
 
-// The tile and K split of least modelled time among tiles [first, last].
-// Each split keeps at least 64 of K, and the partial tiles stay within the
-// staging array of the no-allocation entry point, so both entry points choose alike.
-static void gemm_choose(int64_t M, int64_t N, int64_t K, int64_t batch, bool direct, bool upper, int* tile,
-                        int64_t* splits) {
+// The tile and K split of least modelled time.  Each split keeps at least 64
+// of K, and the partial tiles stay within `room` and the staging array of the
+// no-allocation entry point, so both entry points choose alike.
+static void gemm_choose(int64_t M, int64_t N, int64_t K, int64_t batch, bool direct, bool upper, size_t room,
+                        int* tile, int64_t* splits) {
     static const int S[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512};
     const int cus = device_cus();
+    const int64_t most = (int64_t)std::min<size_t>(room, GEMM_STAGING_MAX);
     double best = 1e300;
     *tile = 3;
     *splits = 1;
@@ -1122,7 +1123,7 @@ static void gemm_choose(int64_t M, int64_t N, int64_t K, int64_t batch, bool dir
         if (!direct && t < 3) continue;                 // unaligned rows: 64 x 64 and 32 x 32 only
         if (upper && GEMM_TILES[t].bm != GEMM_TILES[t].bn) continue;
         for (const int s : S) {
-            if (s > 1 && (K / s < 64 || 8 * s * M * N * batch > GEMM_STAGING_MAX)) break;
+            if (s > 1 && (K / s < 64 || 8 * s * M * N * batch > most)) break;
             const double c = gemm_cost(GEMM_TILES[t], M, N, K, batch, s, upper, cus);
             if (c < best) { best = c; *tile = t; *splits = s; }
         }
@@ -1186,12 +1187,7 @@ static int launch_cfg(xr_ctx* c, int tile, int64_t splits, int ta, int tb, int64
     if (splits > 1) {
         const int64_t need = splits * batch * M * N * (int64_t)sizeof(double);
         Cw = (double*)xr_workspace(c, 50, need);
-        if (!Cw) {             // no room for the partial tiles: unsplit (gemm_admit has let the call through)
-            c->pin_blocked = c->noalloc_blocked = false;
-            splits = 1;
-            kchunk = K;
-            Cw = C;
-        }
+        if (!Cw) return xr_fail(c, XR_ENOMEM, "workspace (split-K)");
     }
     const GemmTile& T = GEMM_TILES[tile];
     const int64_t tm = ceil_div(M, T.bm), tn = ceil_div(N, T.bn), tiles = tm * tn;
@@ -1237,23 +1233,25 @@ static int launch_cfg(xr_ctx* c, int tile, int64_t splits, int ta, int tb, int64
     return XR_OK;
 }
 
-// Refuses a product whose staging (gemm_refusal_bytes) does not fit what
-// the context may hold; remembers the largest that did, as the workspace
-// slot would.
+// Refuses a product whose staging (gemm_refusal_bytes, or a tuned split's) is
+// more than the context may hold.  An admitted one leaves that much behind in the
+// workspace slot, up to the most any split needs: a later product admitted because a larger
+// one ran before the pin then finds room for its own partial tiles.
 static int gemm_admit(xr_ctx* c, int64_t bytes) {
-    if (!(c->pins > 0 || c->ws_limit || c->noalloc)) {
-        if (bytes > c->gemm_staging) c->gemm_staging = bytes;
-        return XR_OK;
+    if (bytes == 0 || (!c->noalloc && bytes <= c->gemm_staging)) return XR_OK;
+    if ((size_t)bytes > xr_workspace_room(c, 50)) {
+        c->noalloc_blocked = c->noalloc;
+        c->pin_blocked = !c->noalloc && c->pins > 0;
+        return xr_fail(c, XR_ENOMEM, "workspace (split-K)");
     }
-    if (bytes == 0 || (!c->noalloc && bytes <= c->gemm_staging) || xr_workspace_fits(c, 50, bytes)) return XR_OK;
-    c->noalloc_blocked = c->noalloc;
-    c->pin_blocked = !c->noalloc && c->pins > 0;
-    return xr_fail(c, XR_ENOMEM, "workspace (split-K)");
+    if (!c->noalloc && xr_workspace(c, 50, std::min(bytes, GEMM_STAGING_MAX))) c->gemm_staging = bytes;
+    return XR_OK;
 }
 
 // One product with the configuration chosen for its sizes, kept in a small
 // direct-mapped table of the context (a pure function of the sizes: an entry
-// never goes stale; at most 1024 of them).
+// never goes stale; at most 1024 of them).  Where a cap leaves less room than its
+// partial tiles take, the best of the splits that fit runs instead.
 static int launch_chosen(xr_ctx* c, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
                          int64_t lda, int64_t sA, const double* B, int64_t ldb, int64_t sB, double beta, double* C,
                          int64_t ldc, int64_t sC, int64_t batch, bool upper = false) {
@@ -1264,13 +1262,18 @@ static int launch_chosen(xr_ctx* c, int ta, int tb, int64_t M, int64_t N, int64_
     if (c->gemm_choice.empty()) c->gemm_choice.resize(1024);
     auto& e = c->gemm_choice[h >> 54];
     if (e.key != key) {
-        gemm_choose(M, N, K, batch, direct, upper, &e.tile, &e.splits);
+        gemm_choose(M, N, K, batch, direct, upper, SIZE_MAX, &e.tile, &e.splits);
         e.staging = gemm_refusal_bytes(M, N, K, beta != 0.0, batch, upper);
         e.key = key;
     }
     const int rc = gemm_admit(c, e.staging);
     if (rc) return rc;
-    return launch_cfg(c, e.tile, e.splits, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch,
+    int tile = e.tile;
+    int64_t splits = e.splits;
+    const size_t room = splits > 1 ? xr_workspace_room(c, 50) : SIZE_MAX;
+    if ((size_t)(8 * splits * M * N * batch) > room)
+        gemm_choose(M, N, K, batch, direct, upper, room, &tile, &splits);
+    return launch_cfg(c, tile, splits, ta, tb, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch,
                       upper);
 }
 

@@ -6,7 +6,9 @@ host, no GPU allocation actually fails):
     again once the cap is lifted;
   * an XRSystem whose sigma budget is below every monomer sigma
     intermediate recomputes them in the adjoint, with the same energy and
-    gradient as the one that stores them."""
+    gradient as the one that stores them;
+  * an FP64 product keeps its K split under a pin that admits it, and under a
+    limit it is refused with its output untouched, or right."""
 import numpy as np
 import pytest
 import torch
@@ -14,6 +16,7 @@ import torch
 from qodeapplications_amd import density as D
 from qodeapplications_amd import synthetic as syn
 from qodeapplications_amd._lib import XR_ENOMEM, XRError, context
+from qodeapplications_amd.gemm import mm
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +61,51 @@ def test_sigma_recomputed_under_budget_matches_stored():
             assert float((z1[m][c] - z2[m][c]).abs().max()) < 1e-10
     for k in i1:
         assert float((i1[k] - i2[k]).abs().max()) < 1e-10
+
+
+def _product(M, N, K, beta=0.0):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    r = lambda a, b: torch.randn(a, b, dtype=torch.float64, device="cuda", generator=g)
+    return r(M, K), r(K, N), r(M, N), beta
+
+
+def test_pinned_product_runs_as_before_the_pin():
+    # a product admitted under a pin because a larger one ran before it keeps
+    # its K split (same bits), though the larger one staged nothing of its own
+    A, B, C, _ = _product(64, 64, 400000)
+    ctx = context(0)
+    ctx.call("xr_trim")
+    want = mm(A, B)
+    ctx.call("xr_trim")
+    a, b, c, beta = _product(2000, 2000, 320, 1.0)
+    mm(a, b, out=c, beta=beta)
+    ctx.call("xr_pin", 1)
+    try:
+        assert torch.equal(mm(A, B), want)
+    finally:
+        ctx.call("xr_pin", -1)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 300, 20000), (64, 65, 100001)])
+def test_product_under_a_limit_is_refused_or_right(M, N, K):
+    A, B, C0, beta = _product(M, N, K, 0.5)
+    ref = A @ B + beta * C0
+    bound = (2 * (K + 2) + 4) * 2.0 ** -53 * (A.abs() @ B.abs() + beta * C0.abs())
+    ctx = context(0)
+    refused = 0
+    limits = [4096] + [8 * M * N * s for s in (1, 2, 3, 5, 8, 13, 21, 34, 55, 89, 144, 233, 377, 610)]
+    try:
+        for limit in limits:
+            ctx.call("xr_trim")
+            ctx.call("xr_set_memory_limit", limit)
+            C = C0.clone()
+            try:
+                mm(A, B, out=C, beta=beta)
+            except XRError as e:
+                assert e.code == XR_ENOMEM and torch.equal(C, C0)
+                refused += 1
+                continue
+            assert bool(((C - ref).abs() <= bound).all()), limit
+    finally:
+        ctx.call("xr_set_memory_limit", 0)
+    assert 0 < refused < len(limits)
