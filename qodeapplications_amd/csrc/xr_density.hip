@@ -1093,6 +1093,13 @@ __global__ void k_sym_sum(const double* __restrict__ G, int64_t n, double* __res
     }
 }
 
+// Whether the scratch of a call's side adjoints, na and nb elements, is there
+// (the larger serves both).
+static bool side_scratch(xr_ctx* c, int64_t na, int64_t nb) {
+    const int64_t n = std::max(na, nb);
+    return n == 0 || xr_workspace(c, WS_ZBT, n * sizeof(double));
+}
+
 static int side_adjoint(xr_ctx* c, const SidePlan& sd, int n_orbs, int n_core, int kspace_core,
                         int n_elec_src, int64_t nK, int64_t nT, const double* Ybar, int64_t nS,
                         int layout, double* zbar, bool add = true) {
@@ -1215,7 +1222,8 @@ static int monomer_2e_adjoint_impl(xr_ctx* c, int n_orbs, int n_core, int n_elec
     double* Wbar = need_wbar ? (double*)xr_workspace(c, WS_WB, szJ) : nullptr;
     double* Veb = Vbar ? (double*)xr_workspace(c, WS_VEB, nU * nU * sizeof(double)) : nullptr;
     if ((need_wbar && !mirror && !X) || (need_y && !Y) || (need_w && (!W || !Xbar)) ||
-        (zbar_ket && !mirror && !Ybar) || (need_wbar && !Wbar) || (Vbar && !Veb))
+        (zbar_ket && !mirror && !Ybar) || (need_wbar && !Wbar) || (Vbar && !Veb) ||
+        !side_scratch(c, zbar_bra ? nP * nI : 0, zbar_ket && !mirror ? nQ * nJ : 0))
         return xr_fail(c, XR_ENOMEM, "workspace (sigma adjoint)");
     Coeffs cb, ck;
     if ((rc = coeffs_for_gather(c, WS_ZTB, WS_ZTK, nI, nP, X ? zbra : nullptr, nJ, nQ, Y ? zket : nullptr, &cb, &ck)))
@@ -1252,19 +1260,16 @@ static int monomer_2e_adjoint_impl(xr_ctx* c, int n_orbs, int n_core, int n_elec
     if (need_wbar && (rc = xr_gemm_2e(c, 0, 0, Kp * nK, nJ, nI, mirror ? sg : 1.0, mirror ? Y : X, nI, 0, Ebar, nJ, 0,
                                       0.0, Wbar, nJ, 0, 1)))
         return rc;
+    // every product before the first output is added to: a call that is refused
+    // memory (a limit, a pin) leaves all outputs as they were
+    // Veb = Wbar Y^T (nU x nU), Ybar = Ve^T Wbar (nU x KJ)
+    if (Vbar && (rc = xr_gemm_2e(c, 0, 1, nU, nU, KJ, 1.0, Wbar, KJ, 0, Y, KJ, 0, 0.0, Veb, nU, 0, 1))) return rc;
+    if (Ybar && (rc = veff_product(c, V, nullptr, 0.0, dim, true, Wbar, KJ, Ybar))) return rc;
     if (Vbar) {
-        // Veb = Wbar Y^T (nU x nU), then scatter into Vbar
-        if ((rc = xr_gemm_2e(c, 0, 1, nU, nU, KJ, 1.0, Wbar, KJ, 0, Y, KJ, 0, 0.0, Veb, nU, 0, 1)))
-            return rc;
         k_veff_adjoint<<<xr_grid(nU * nU), 256, 0, c->stream>>>(Veb, dim, nU, Vbar);
         XR_LAUNCH_CHECK(c);
     }
-    if (Ybar) {
-        // Ybar = Ve^T Wbar (nU x KJ)
-        if ((rc = veff_product(c, V, nullptr, 0.0, dim, true, Wbar, KJ, Ybar))) return rc;
-        if ((rc = side_adjoint(c, pl.R, n_orbs, n_core, 0, n_elec, nK, nU, Ybar, nJ, 2, zbar_ket)))
-            return rc;
-    }
+    if (Ybar && (rc = side_adjoint(c, pl.R, n_orbs, n_core, 0, n_elec, nK, nU, Ybar, nJ, 2, zbar_ket))) return rc;
     if (zbar_bra && (rc = side_adjoint(c, pl.L, n_orbs, n_core, 0, n_elec, nK, nU, Xbar, nI, 2, zbar_bra)))
         return rc;
     return XR_OK;
@@ -1353,7 +1358,8 @@ extern "C" int xr_density_adjoint(xr_ctx* c, const char* ops, int n_orbs, int n_
                         nP == nQ && Mg == Ng && zbar_bra == zbar_ket && zbar_ket && pl.R.k;
     double* Xbar = zbar_bra && !mirror && pl.L.k ? (double*)xr_workspace(c, WS_XB, f.nK * Mg * sizeof(double)) : nullptr;
     double* Ybar = zbar_ket && pl.R.k ? (double*)xr_workspace(c, WS_YB, f.nK * Ng * sizeof(double)) : nullptr;
-    if (!Gc || (zbar_bra && !mirror && pl.L.k && !Xbar) || (zbar_ket && pl.R.k && !Ybar))
+    if (!Gc || (zbar_bra && !mirror && pl.L.k && !Xbar) || (zbar_ket && pl.R.k && !Ybar) ||
+        !side_scratch(c, Xbar ? nP * nI : 0, Ybar ? nQ * nJ : 0))
         return xr_fail(c, XR_ENOMEM, "workspace (adjoint)");
     {
         int64_t n = Mg * Ng;
@@ -1380,33 +1386,26 @@ extern "C" int xr_density_adjoint(xr_ctx* c, const char* ops, int n_orbs, int n_
         return side_adjoint(c, pl.R, n_orbs, n_core, f.kspace_core, n_elec_ket, f.nK, f.nT, Ybar, nJ, 0,
                             zbar_ket);
     }
-    if (zbar_ket) {
-        if (pl.R.k) {
-            // Ybar = X Gc  (nK x Ng), then the transpose of the gather
-            if ((rc = xr_dgemm_launch(c, f.xT, 0, f.nK, Ng, Mg, 1.0, f.X, f.ldx, 0, Gc, Ng, 0, 0.0, Ybar, Ng, 0, 1)))
-                return rc;
-            if ((rc = side_adjoint(c, pl.R, n_orbs, n_core, f.kspace_core, n_elec_ket, f.nK, f.nT, Ybar, nJ, 0,
+    // Every product that can be refused memory (a limit, a pin) and every read of
+    // the coefficients comes before the first output is added to.
+    // Ybar = X Gc (nK x Ng), Xbar = Y Gc^T (nK x Mg)
+    if (Ybar && (rc = xr_dgemm_launch(c, f.xT, 0, f.nK, Ng, Mg, 1.0, f.X, f.ldx, 0, Gc, Ng, 0, 0.0, Ybar, Ng, 0, 1)))
+        return rc;
+    if (Xbar && (rc = xr_dgemm_launch(c, f.yT, 1, f.nK, Mg, Ng, 1.0, f.Y, f.ldy, 0, Gc, Ng, 0, 0.0, Xbar, Mg, 0, 1)))
+        return rc;
+    // without R, Y = zket^T: zbar_ket (nJ x nQ) += Gc^T X^T; without L, X = zbra^T:
+    // zbar_bra (nI x nP) += Gc Y^T
+    if (zbar_ket && !pl.R.k &&
+        (rc = xr_dgemm_launch(c, 1, 1, nJ, nQ, Mg, 1.0, Gc, Ng, 0, f.X, f.ldx, 0, 1.0, zbar_ket, nQ, 0, 1)))
+        return rc;
+    if (zbar_bra && !pl.L.k &&
+        (rc = xr_dgemm_launch(c, 0, 1, nI, nP, Ng, 1.0, Gc, Ng, 0, f.Y, f.ldy, 0, 1.0, zbar_bra, nP, 0, 1)))
+        return rc;
+    // then the transposes of the gathers
+    if (Ybar && (rc = side_adjoint(c, pl.R, n_orbs, n_core, f.kspace_core, n_elec_ket, f.nK, f.nT, Ybar, nJ, 0,
                                    zbar_ket)))
-                return rc;
-        } else {
-            // Y = zket^T: zbar_ket (nJ x nQ) += Gc^T X^T
-            if ((rc = xr_dgemm_launch(c, 1, 1, nJ, nQ, Mg, 1.0, Gc, Ng, 0, f.X, f.ldx, 0, 1.0, zbar_ket, nQ, 0, 1)))
-                return rc;
-        }
-    }
-    if (zbar_bra) {
-        if (pl.L.k) {
-            // Xbar = Y Gc^T  (nK x Mg)
-            if ((rc = xr_dgemm_launch(c, f.yT, 1, f.nK, Mg, Ng, 1.0, f.Y, f.ldy, 0, Gc, Ng, 0, 0.0, Xbar, Mg, 0, 1)))
-                return rc;
-            if ((rc = side_adjoint(c, pl.L, n_orbs, n_core, f.kspace_core, nb, f.nK, f.nLt, Xbar, nI, 0,
-                                   zbar_bra)))
-                return rc;
-        } else {
-            // X = zbra^T: zbar_bra (nI x nP) += Gc Y^T
-            if ((rc = xr_dgemm_launch(c, 0, 1, nI, nP, Ng, 1.0, Gc, Ng, 0, f.Y, f.ldy, 0, 1.0, zbar_bra, nP, 0, 1)))
-                return rc;
-        }
-    }
+        return rc;
+    if (Xbar && (rc = side_adjoint(c, pl.L, n_orbs, n_core, f.kspace_core, nb, f.nK, f.nLt, Xbar, nI, 0, zbar_bra)))
+        return rc;
     return XR_OK;
 }

@@ -8,14 +8,15 @@ host, no GPU allocation actually fails):
     intermediate recomputes them in the adjoint, with the same energy and
     gradient as the one that stores them;
   * an FP64 product keeps its K split under a pin that admits it, and under a
-    limit it is refused with its output untouched, or right."""
+    limit it is refused with its output untouched, or right;
+  * an adjoint that is refused at any limit has added to none of its outputs."""
 import numpy as np
 import pytest
 import torch
 
 from qodeapplications_amd import density as D
 from qodeapplications_amd import synthetic as syn
-from qodeapplications_amd._lib import XR_ENOMEM, XRError, context
+from qodeapplications_amd._lib import XR_ENOMEM, XRError, context, ptr
 from qodeapplications_amd.gemm import mm
 
 pytestmark = pytest.mark.gpu
@@ -109,3 +110,46 @@ def test_product_under_a_limit_is_refused_or_right(M, N, K):
     finally:
         ctx.call("xr_set_memory_limit", 0)
     assert 0 < refused < len(limits)
+
+
+@pytest.mark.parametrize("op", ["a", "aa", "c", "cc", "ca", "caa", "cca", "2e"])
+def test_refused_adjoint_leaves_its_outputs(op):
+    n, ne, nI, nJ = 6, 4, 7, 4
+    nb = ne if op == "2e" else ne + op.count("c") - op.count("a")
+    rng = np.random.default_rng(4)
+    kb = D.ChargeBlock.from_states(syn.random_states(n, ne, nJ, rng), n, 0)
+    bb = D.ChargeBlock.from_states(syn.random_states(n, nb, nI, rng), n, 0)
+    dim = 2 * n
+    rand = lambda *s: torch.as_tensor(rng.standard_normal(s), device="cuda")
+    head = (n, 0, ne, nI, bb.n_configs, ptr(bb.coeffs), nJ, kb.n_configs, ptr(kb.coeffs))
+    init = [rand(*bb.coeffs.shape), rand(*kb.coeffs.shape)]
+    if op == "2e":
+        V, Eb = rand(dim, dim, dim, dim), rand(nI, nJ)
+        init.append(rand(dim, dim, dim, dim))
+        call = lambda out: context(0).call("xr_monomer_2e_adjoint", *head, ptr(V), ptr(Eb), *[ptr(t) for t in out])
+    else:
+        Rb = rand(nI, nJ, *([dim] * len(op)))
+        call = lambda out: context(0).call("xr_density_adjoint", op.encode(), *head, ptr(Rb), *[ptr(t) for t in out])
+    want = [t.clone() for t in init]
+    call(want)
+    ctx = context(0)
+    limit, refused = 2048, 0
+    try:
+        while True:
+            ctx.call("xr_trim")
+            ctx.call("xr_set_memory_limit", int(limit))
+            out = [t.clone() for t in init]
+            try:
+                call(out)
+                break
+            except XRError as e:
+                assert e.code == XR_ENOMEM
+                assert all(torch.equal(a, b) for a, b in zip(out, init)), limit
+                refused += 1
+                limit *= 1.05
+    finally:
+        ctx.call("xr_set_memory_limit", 0)
+    assert refused > 0
+    # not the same bits: a limit may leave a product another split of K
+    for a, b in zip(out, want):
+        assert float((a - b).abs().max()) < 1e-12 * float(b.abs().max())
