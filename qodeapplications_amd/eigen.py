@@ -158,11 +158,13 @@ def lowest_root(A):
     cap = min(n, max(160, n // 4))
     V = torch.empty(cap, n, dtype=torch.float64, device=A.device)
     work = torch.empty(4 * cap + 128 + 2 * n, dtype=torch.float64, device=A.device)
-    ctx = context(A.device.index)
+    # bound to the current stream again for every call: the host reads in between
+    # let other threads bind the shared context to theirs
+    call = lambda *args: context(A.device.index).call(*args)
     u, nb = 2.0 ** -53, -(-n // 64)
     done, m, looks = 0, LANCZOS_FIRST, []
     while m <= cap:
-        ctx.call("xr_lanczos_steps", n, ptr(A), n, done, m, cap, ptr(V), n, ptr(work))
+        call("xr_lanczos_steps", n, ptr(A), n, done, m, cap, ptr(V), n, ptr(work))
         done = m
         h = work[:2 * cap + nb].cpu().numpy()
         beta = np.append(h[cap + 1:cap + m], np.sqrt(h[2 * cap:].sum()))
@@ -176,7 +178,8 @@ def lowest_root(A):
         est = beta[k - 1] * t[2]
         if est <= u * t[1] or k < m:
             v = torch.empty(n, 1, dtype=torch.float64, device=A.device)
-            ctx.call("xr_lanczos_root", n, ptr(A), n, k, cap, ptr(V), n, ptr(upload(t[3], A.device)), ptr(work), ptr(v))
+            s = upload(t[3], A.device)
+            call("xr_lanczos_root", n, ptr(A), n, k, cap, ptr(V), n, ptr(s), ptr(work), ptr(v))
             w = work[:2].clone()
             if float(w[1]) <= 16 * u * t[1]:
                 return w[:1], v
