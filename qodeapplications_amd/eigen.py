@@ -168,8 +168,9 @@ def lowest_root(A):
         done = m
         h = work[:2 * cap + nb].cpu().numpy()
         beta = np.append(h[cap + 1:cap + m], np.sqrt(h[2 * cap:].sum()))
-        # an invariant subspace: what follows a vanished coupling is noise
-        scale = max(np.abs(h[:m]).max(), beta.max())
+        # an invariant subspace: a coupling that vanishes against all before it (what
+        # follows is normalised noise, of any size)
+        scale = np.maximum.accumulate(np.maximum(np.abs(h[:m]), np.append(0.0, beta[:-1])))
         cut = np.flatnonzero(~(beta > n * u * scale))
         k = int(cut[0]) + 1 if len(cut) else m
         t = _tridiag_lowest(h[:k].copy(), beta[:k].copy())

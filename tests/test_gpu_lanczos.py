@@ -55,6 +55,21 @@ def test_lowest_root(kind, n):
     assert torch.equal(w, w2) and torch.equal(v, v2)
 
 
+@pytest.mark.parametrize("kind", ["gap", "projector"])
+@pytest.mark.parametrize("n", [128, 129, 577, 1030])
+def test_iterates_without_the_full_decomposition(kind, n, monkeypatch):
+    M = torch.as_tensor(_matrix(kind, n, np.random.default_rng(n)), device="cuda")
+    ref = torch.linalg.eigvalsh(M)
+
+    def eigh(*a, **k):
+        raise AssertionError("fell back to the full decomposition")
+
+    monkeypatch.setattr(torch.linalg, "eigh", eigh)
+    w, v = eigen.lowest_root(M)
+    nrm = float(ref.abs().max())
+    assert abs(float(w[0] - ref[0])) <= 32 * U * nrm + 4 * n * U * nrm
+
+
 def test_context_bound_elsewhere_between_the_host_reads(monkeypatch):
     # what another thread's call does while this one waits for the device
     M = torch.as_tensor(_matrix("gap", 577, np.random.default_rng(1)), device="cuda")
