@@ -237,9 +237,10 @@ int xr_gemm_f64_noalloc(xr_ctx *ctx, int transA, int transB, int64_t M, int64_t 
 
 /* n independent products C_q = alpha op(A_q) op(B_q) of uneven shapes
  * (host arrays of n shapes, leading dimensions and device pointers; the same
- * transposes for all), their output tiles in one grid per 24 problems of one
- * tile shape (tall-skinny products go to the single-product kernels);
- * every C_q is overwritten.  Used for the pair-term products of one XR
+ * transposes for all), their output tiles in one grid per 32 problems of one
+ * tile shape and alignment, or of all of them where the tiles are few
+ * (tall-skinny products go to the single-product kernels); every C_q is
+ * overwritten.  Used for the pair-term products of one XR
  * operator application (general-XRCC/hamiltonian.py:21-63, the pair terms
  * H2_mn (x) 1 of all charge groups at once). */
 int xr_gemm_grouped(xr_ctx *ctx, int n, int transA, int transB, const int64_t *M, const int64_t *N,

@@ -434,9 +434,8 @@ int xr_space_masks(xr_ctx* c, int n_orbs, int n_core, int n_elec, const uint64_t
 struct Coeffs { const double* z; int64_t sC, sS; };
 
 // Up to this many bytes of coefficients are gathered as they are stored, which
-// saves the transposing launch.  With both gathers in one launch, a small product in
-// one piece and the tiled expansion, ca of 9 orbitals, 3 electrons, 8 x 8 states: 21.9 -> 15.6 us
-// (together; not measured apart).
+// saves the transposing launch: ca of 9 orbitals, 3 electrons, 8 x 8 states, 18.9 us
+// with it, 15.8 without (both gathers in one launch save 0.4 us of that, within the spread).
 #define GATHER_DIRECT_BYTES (1 << 20)
 
 // The two blocks' coefficients for a gather, those of size > GATHER_DIRECT_BYTES

@@ -18,6 +18,8 @@ typedef double d2_t __attribute__((ext_vector_type(2)));
 
 #define GEMM_BK 16
 #define GEMM_THREADS 256
+// s_waitcnt operand: vmcnt 0, the other counters unlimited
+#define GEMM_WAIT_VMCNT0 0x0F70
 // output row of accumulator element r for lane group fk (lane / 16) of
 // v_mfma_f32_16x16x4f32 (checked on gfx950; the f64 variant differs)
 #define XR_F32_ROW(fk, r) (4 * (fk) + (r))
@@ -194,10 +196,10 @@ struct TileFrags {
 // that ends the previous step, all fragment reads of this stage, then the
 // loads of the next stage (after the reads: the compiler makes a read wait
 // for every load into LDS queued before it), then the MFMAs.  The accumulators live
-// in ordinary registers (220 of 256 at two waves per SIMD), so alpha and beta
-// cost nothing at the store.  Measured on 8192^3: 73.4 TFLOP/s (0.93 of
-// the FP64 matrix peak), against 59.7 with guarded 8-byte loads through
-// registers and two barriers per step.
+// in ordinary registers (220 to 244 of 256 at two waves per SIMD), so alpha and beta
+// cost nothing at the store.  Measured on 8192^3: 71.5 to 72.7 TFLOP/s by
+// transposes (0.91 to 0.925 of the FP64 matrix peak), against 59.7 with guarded
+// 8-byte loads through registers and two barriers per step.
 // Fragments wholly past M or N are skipped, and neighbouring fragments
 // belong to different waves, so an edge tile costs about its valid 16 or 32 row
 // groups on every SIMD rather than the whole tile.
@@ -282,7 +284,11 @@ __device__ __forceinline__ void dgemm_tile(int64_t M, int64_t N, int64_t K, doub
         }
     };
     auto step = [&](auto FULL, int cur, int tnext) {
-        __syncthreads();                       // this stage is in LDS, the other one is free
+        // this wave's loads into LDS have landed (vmcnt 0: a barrier waits for
+        // its waves, not for their loads); after the barrier every wave's have, and the
+        // other stage is free
+        if constexpr (DIRECT) __builtin_amdgcn_s_waitcnt(GEMM_WAIT_VMCNT0);
+        __syncthreads();
         if constexpr (DIRECT) {
 #pragma unroll
             for (int s = 0; s < GEMM_BK / 8; s++) {
@@ -1064,11 +1070,14 @@ static int launch_nn_gram(xr_ctx* c, int64_t M, int64_t N, int64_t K, double alp
 // ---------------------------------------------------------------------------
 // Tile 0: 128 x 128, 1: 128 x 64, 2: 64 x 128, 3: 64 x 64, 4: 32 x 32 (k_dgemm_small).
 struct GemmTile { int bm, bn, resident; double eff, alone; };
-// resident: workgroups a CU holds; eff: share of the FP64 matrix peak with
-// the CU full; alone: us one 16-deep step takes over its MFMAs when a
-// workgroup has the CU to itself (load latency and the barrier).  Measured
-// on products of 64 x 324 x 64 to 8192^3 (68.8, 68.3, 68.1 and 66.4 TFLOP/s for tiles 0 to 3 on
-// 8192 x 8192 x 4096; 142, 80, 79 and 47 us for 64, 128, 128 and 256 workgroups of 1024^3).
+// resident: workgroups the model takes a CU to hold; eff: share of the FP64
+// matrix peak with the CU full; alone: us one 16-deep step takes over its
+// MFMAs when a workgroup has the CU to itself (load latency and the barrier).  Set from
+// products of 64 x 324 x 64 to 8192^3; measured at rest on 8192 x 8192 x 4096: 72.2, 71.5, 71.7 and 71.3
+// TFLOP/s for tiles 0 to 3 (0.91 to 0.92 of the peak, so eff is a little low for all alike), and
+// 137, 75, 76 and 45 us for 64, 128, 128 and 256 workgroups of 1024^3.  By their registers the 64 x 64
+// kernels of unaligned rows with B transposed hold four workgroups, and the 32 x 32
+// one two, unless B alone is transposed: past that many the wait is modelled too short.
 static const GemmTile GEMM_TILES[5] = {
     {128, 128, 2, 0.90, 0.50}, {128, 64, 3, 0.89, 0.40}, {64, 128, 3, 0.89, 0.40}, {64, 64, 5, 0.87, 0.26}, {32, 32, 4, 0.60, 0.10}};
 #define GEMM_STAGING_MAX ((int64_t)64 << 20)   // bytes of split-K partial tiles
@@ -1549,7 +1558,7 @@ extern "C" int xr_gemm_grouped(xr_ctx* c, int n, int ta, int tb, const int64_t* 
         tiles += ceil_div(M[q], 64) * ceil_div(N[q], 64);
         direct = direct && gemm_direct(ta, tb, M[q], N[q], K[q], A[q], lda[q], 0, B[q], ldb[q], 0);
     }
-    if (!all.empty() && tiles <= 2 * 256)
+    if (!all.empty() && tiles <= 2 * device_cus())
         return direct ? launch_grouped<64, 64>(c, all, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc)
                       : launch_grouped<64, 64, false>(c, all, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc);
     int rc = launch_grouped_any<128, 128>(c, wide, ta, tb, M, N, K, alpha, A, lda, B, ldb, C, ldc);

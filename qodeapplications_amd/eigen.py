@@ -142,7 +142,9 @@ def lowest_root(A):
     """(values[1], vectors[n, 1]) of the symmetric device matrix A: Lanczos to
     a residual at the rounding of A's norm, checked on the vector itself, and
     the full eigendecomposition where it does not get there (a gap too narrow
-    for the steps allowed, entries that are not finite) or would not pay.
+    for the steps allowed, entries that are not finite) or would not pay.  The
+    vector of an exactly degenerate root is the start vector's part in its
+    eigenspace (the same bits on every run), not the full decomposition's choice.
 
     Against the full one, XR matrices of 256 / 576 / 1296 rows: 6.2 / 13.3 / 29.8 ms
     -> 1.2 / 1.6 / 2.1, residuals of 2e-16 to 5e-16 |A| for 6e-16 to 1.2e-15; 128 rows

@@ -48,8 +48,8 @@ class Hamiltonian:
         if tuple(self.h.shape) != (dim, dim) or tuple(self.V.shape) != (dim,) * 4:
             raise ValueError(f"h must be {dim} x {dim} and V {dim}^4")
         self.n_configs = self.configs.shape[0]
-        self._block = ChargeBlock(self.n_orbs, self.n_core, self.configs,
-                                  np.zeros((1, self.n_configs)), device=dev)
+        # refuses a space the library does not take before any sigma is asked for
+        ChargeBlock(self.n_orbs, self.n_core, self.configs, np.zeros((0, self.n_configs)), device=dev)
         self._diag = None
 
     def sigma(self, Z, chunk=64):
