@@ -1483,7 +1483,8 @@ static int launch_grouped(xr_ctx* c, const std::vector<int>& ids, int ta, int tb
         }
         if (8 * slots > 0x7fffffff) return xr_fail(c, XR_EUNSUPPORTED, "GEMM grid too large");
         ProfScope prof(c, kind, flops, bytes);
-        prof.shape(g.p[0].M, g.p[0].N, g.p[0].K, g.n, ta, tb);
+        // no shape in the class of the single products: the tuner would time it as one
+        if (kind != XR_K_GEMM_F64) prof.shape(g.p[0].M, g.p[0].N, g.p[0].K, g.n, ta, tb);
         const dim3 grid((unsigned)(8 * slots));
 #define XR_GROUPED(TA_, TB_) \
     k_dgemm_grouped<BM, BN, TA_, TB_, DIRECT><<<grid, GEMM_THREADS, 0, c->stream>>>(g)

@@ -17,6 +17,7 @@ from qodeapplications_amd import density as D
 from qodeapplications_amd import synthetic as syn
 from qodeapplications_amd._lib import context, ptr
 from qodeapplications_amd.fci import Hamiltonian
+from qodeapplications_amd.graph import gemm_shapes
 from qodeapplications_amd.xr import precision
 
 pytestmark = pytest.mark.gpu
@@ -100,6 +101,14 @@ def test_sigma_equals_the_adjoints(n_orbs, n_elec, n_core, nv, mix):
     terms = dim * (dim - 1) // 2 + dim + n_elec ** 2 + 16
     bound = 2 * terms * U * _abs_sigma(H, Z) + 1e-300
     assert bool(((got - ref).abs() <= bound).all()), float(((got - ref).abs() / bound).max())
+
+
+def test_the_tuner_sees_single_products_only():
+    # the class blocks are one grouped launch, no product of a shape to be tuned
+    h, V = _integrals(13, 3, False)
+    kb = D.ChargeBlock.from_states(syn.random_states(13, 5, 2, np.random.default_rng(0)), 13, 0)
+    pairs, rest = 26 * 25 // 2, 2600
+    assert gemm_shapes(lambda: D.monomer_2e(kb, kb, V)).keys() <= {(1, 0, 2, 2, pairs * rest, 1)}
 
 
 @pytest.mark.parametrize("mode", ["split_f32", "split_i8"])
