@@ -69,7 +69,8 @@ int xr_pin(xr_ctx *ctx, int delta);
 
 /* Caps the total bytes of the context's workspaces (0 = no cap): a call
  * whose scratch would exceed it fails with XR_ENOMEM instead of allocating
- * (for callers that share HBM with other work; also how the out-of-memory
+ * (the density and two-electron adjoints then have added to none of their outputs;
+ * for callers that share HBM with other work; also how the out-of-memory
  * paths are tested).  No reference counterpart. */
 int xr_set_memory_limit(xr_ctx *ctx, int64_t bytes);
 
